@@ -2,6 +2,7 @@
 // buffers, per-frame orchestration of the kernels in er_kernels.h.
 #include "er_capi.h"
 #include "er_kernels.h"
+#include "er_linefft.h"
 
 #include <hip/hip_runtime.h>
 
@@ -20,7 +21,7 @@ namespace {
 
 constexpr int NI_B = 16;  // insertion interleave of the batched path
 constexpr int ER_KSLICES = 16;  // insertion slices of the split-K edens/ecorr sums
-constexpr int ER_SPARSE_SITES = 12;  // above this many sites the plane kernel spreads + transforms
+constexpr int ER_SPARSE_SITES = ER_DENSE_SITES;  // above this many sites the plane kernel spreads + transforms
 
 // device buffer owned by one context (freed with it); movable, not copyable
 template <typename T> struct DBuf {
@@ -178,6 +179,10 @@ struct er_ctx {
     DBuf<double> d_splfc1, d_splfc2, d_splfc3;
     DBuf<float> d_engfac;
     DBuf<float2> d_tw1, d_tw2, d_tw3, d_twm, d_tws;
+    // lengths without a compiled kernel: factors and position tables (nf = 0:
+    // a prime factor above 7, the direct kernels)
+    LinePlan lp[3] = {};
+    DBuf<unsigned short> d_rev[3];
     DBuf<double> d_selfpart;
     DBuf<float2> d_Ftab;           // per-insertion separable structure-factor factors
     DBuf<float2> d_T;
@@ -358,6 +363,54 @@ static bool fft_len_ok(int n)
 
 // (K2, K3) plane shapes with a compiled plane kernel
 static bool plane_ok(int k2, int k3) { return (k2 == k3 && fft_len_ok(k2)) || (k2 == 128 && k3 == 108); }
+
+static unsigned int div_magic(int d) { return d > 1 ? (unsigned int)((0x100000000ull + d - 1) / d) : 0u; }
+
+// the factors of a line of length n for er_linefft.h: the fewest passes, then
+// the smallest largest radix; rev: where natural index k sits in the
+// transform's own order.  False: no such factors.
+static bool line_plan(int n, LinePlan &pl, std::vector<unsigned short> &rev)
+{
+    static const int radix[] = {2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 15, 16};
+    pl = LinePlan{};
+    pl.N = n;
+    int best = 1 << 30;
+    auto take = [&](int nf, int a, int b, int c) {
+        const int score = nf * 64 + std::max(a, std::max(b, c));
+        if (score >= best) return;
+        best = score;
+        pl.nf = nf;
+        pl.R[0] = a;
+        pl.R[1] = b;
+        pl.R[2] = c;
+    };
+    for (int a : radix) {
+        if (a == n) take(1, a, 1, 1);
+        for (int b : radix) {
+            if (a * b == n) take(2, a, b, 1);
+            for (int c : radix)
+                if (a * b * c == n) take(3, a, b, c);
+        }
+    }
+    if (!pl.nf) return false;
+    int len = n;
+    for (int i = 0; i < pl.nf; ++i) {
+        pl.sub[i] = len / pl.R[i];
+        pl.tstep[i] = n / len;
+        pl.msub[i] = div_magic(pl.sub[i]);
+        len = pl.sub[i];
+    }
+    rev.resize(n);
+    for (int k = 0; k < n; ++k) {
+        int at = 0, q = k;
+        for (int i = 0; i < pl.nf; ++i) {
+            at += (q % pl.R[i]) * pl.sub[i];
+            q /= pl.R[i];
+        }
+        rev[k] = (unsigned short)at;
+    }
+    return true;
+}
 
 // cardinal B-spline M_n (spline.F90:46-58) in double for the |b|^2 factors
 static double mn_spline(int n, double x)
@@ -641,6 +694,12 @@ extern "C" int er_create(const er_topology *topo, const er_params *prm, er_ctx *
     HIPCHK(c, upload_tw(c->d_tw2, c->K2, s));
     HIPCHK(c, upload_tw(c->d_tw3, c->K3, s));
     HIPCHK(c, upload_tw(c->d_twm, c->K1 / 2, s));
+    for (int d = 0; d < 3; ++d) {
+        std::vector<unsigned short> rev;
+        if (!line_plan(prm->ms[d], c->lp[d], rev)) continue;
+        HIPCHK(c, c->d_rev[d].ensure(rev.size()));
+        HIPCHK(c, hipMemcpy(c->d_rev[d].p, rev.data(), rev.size() * sizeof(unsigned short), hipMemcpyHostToDevice));
+    }
     {
         std::vector<float2> t(ER_TWS_TOTAL);
         for (int r = 4; r <= 16; ++r)
@@ -1177,7 +1236,45 @@ template <int K2, int K3> static hipError_t launch_spec2d_k(er_ctx *c, int n_off
     return hipGetLastError();
 }
 
-// the direct-DFT plane kernel for shapes without a compiled one
+// Planes without a compiled kernel.  Lengths of small prime factors take the
+// factored kernel (k_pme_spec2d_mix), the others the direct one: on 60 x 60 x
+// 100 with 300 insertions of nine sites stage A measured 412 us against 3850 us
+// direct, on 45 x 50 x 75 with 101 insertions of 25 sites 264 us against
+// 911 us.  Threads per plane: the count that leaves the fewest of a pass's
+// lanes idle.
+static hipError_t launch_spec2d_mix(er_ctx *c, int n_off, int nch, int t_off, bool sparse)
+{
+    static bool attr = false;
+    if (!attr) {
+        (void)hipFuncSetAttribute((const void *)k_pme_spec2d_mix, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  160 * 1024);
+        attr = true;
+    }
+    const int K2 = c->K2, K3 = c->K3;
+    int nt = 512;
+    double best = 1e30;
+    for (int t = 512; t >= 256; t -= 64) {
+        double slots = 0.0;  // thread slots (by the work of one) the passes occupy
+        for (int d = 1; d < 3; ++d)
+            for (int i = 0; i < c->lp[d].nf; ++i) {
+                const int items = K2 * K3 / c->lp[d].R[i];
+                slots += (double)((items + t - 1) / t) * t * (c->lp[d].R[i] + 4);
+            }
+        if (slots < 0.97 * best) {
+            best = slots;
+            nt = t;
+        }
+    }
+    float2 *T = c->d_T.p + (size_t)(n_off - t_off) * c->Gc;
+    hipLaunchKernelGGL(k_pme_spec2d_mix, dim3(c->H, nch), dim3(nt), spec2d_mix_lds(K2, K3), c->stream,
+                       (int)c->plan.desc.size(), c->d_sd.p, c->ord, c->K1, K2, K3, c->lp[1], c->lp[2],
+                       div_magic(K2), div_magic(K3), c->d_rev[1].p, c->d_rev[2].p, (int)sparse, n_off, c->d_Ftab.p,
+                       c->d_insw.p, c->d_insg.p, c->d_engfac.p, c->d_tw2.p, c->d_tw3.p, c->d_tws.p, T,
+                       c->d_selfpart.p);
+    return hipGetLastError();
+}
+
+// the direct-DFT plane kernel
 static hipError_t launch_spec2d_gen(er_ctx *c, int n_off, int nch, int t_off, bool sparse)
 {
     static bool attr = false;
@@ -1198,7 +1295,9 @@ static hipError_t launch_spec2d_gen(er_ctx *c, int n_off, int nch, int t_off, bo
 static hipError_t launch_spec2d(er_ctx *c, int n_off, int nch, int t_off, bool sparse)
 {
     if (nch <= 0) return hipSuccess;
-    if (!plane_ok(c->K2, c->K3)) return launch_spec2d_gen(c, n_off, nch, t_off, sparse);
+    if (!plane_ok(c->K2, c->K3))
+        return c->lp[1].nf && c->lp[2].nf ? launch_spec2d_mix(c, n_off, nch, t_off, sparse)
+                                          : launch_spec2d_gen(c, n_off, nch, t_off, sparse);
     if (c->K2 == c->K3) {
         switch (c->K2) {
         case 32: return launch_spec2d_k<32, 32>(c, n_off, nch, t_off, sparse);
@@ -1257,6 +1356,25 @@ template <int K1, int NI> static hipError_t launch_axis1_k(er_ctx *c, int nch)
 
 template <int NI> static hipError_t launch_axis1(er_ctx *c, int nch)
 {
+    if (!fft_len_ok(c->K1) && NI == 16 && c->lp[0].nf) {
+        // the factored kernel: the most lines per workgroup (64-byte runs of T
+        // at eight) whose LDS still leaves three workgroups per CU.  60 x 60 x
+        // 100, 300 insertions: 258 us (3.4 TB/s over T and phi) against 681 us direct.
+        int rsh = 3;
+        while (rsh > 0 && axis1_mix_lds(c->K1, 1 << rsh) > 53 * 1024) --rsh;
+        static bool attr = false;
+        if (!attr) {
+            (void)hipFuncSetAttribute((const void *)k_pme_axis1_mix, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      160 * 1024);
+            attr = true;
+        }
+        const int nline = c->K2 * c->K3, RL = 1 << rsh;
+        const long nblk = (long)((nline + RL - 1) / RL) * ((nch + 15) / 16);
+        hipLaunchKernelGGL(k_pme_axis1_mix, dim3((unsigned)(8 * ((nblk + 7) / 8))), dim3(256),
+                           axis1_mix_lds(c->K1, RL), c->stream, nch, c->K1, nline, rsh, c->lp[0], div_magic(RL * 8),
+                           c->d_rev[0].p, c->d_T.p, c->d_phi.p, c->d_tw1.p, c->d_tws.p);
+        return hipGetLastError();
+    }
     if (!fft_len_ok(c->K1)) {  // the direct C2R kernel
         const int ntile = (nch + NI - 1) / NI;
         const size_t lds = ((size_t)NI * c->H + c->K1) * sizeof(float2);
@@ -2751,6 +2869,7 @@ extern "C" void er_destroy(er_ctx *c)
     c->d_insposn.release(); c->d_insposu.release(); c->d_insref.release(); c->d_insw.release(); c->d_selfreal.release(); c->d_insg.release();
     c->d_splfc1.release(); c->d_splfc2.release(); c->d_splfc3.release(); c->d_engfac.release();
     c->d_tw1.release(); c->d_tw2.release(); c->d_tw3.release(); c->d_twm.release(); c->d_tws.release();
+    for (auto &r : c->d_rev) r.release();
     c->d_selfpart.release(); c->d_Ftab.release(); c->d_T.release(); c->d_phi.release();
     c->d_C.release(); c->d_w.release(); c->d_border.release(); c->d_bdesc.release(); c->d_flceng.release(); c->d_part.release(); c->d_epart.release();
     if (c->stream2) (void)hipStreamSynchronize(c->stream2);

@@ -94,6 +94,45 @@ template <int SIGN> struct Dft<5, SIGN> {
     }
 };
 
+// radix 7 by the symmetric pairs v_t +- v_{7-t}: three cosine sums and three
+// sine sums of the pairs
+template <int SIGN> struct Dft<7, SIGN> {
+    __device__ __forceinline__ static void run(float2 *v)
+    {
+        const float c[3] = {0.623489801858733530525004884004239811f,    // cos(2 pi/7)
+                            -0.222520933956314404288902564496794760f,   // cos(4 pi/7)
+                            -0.900968867902419126236102319507445051f};  // cos(6 pi/7)
+        const float s[3] = {0.781831482468029808708444526674057750f,    // sin(2 pi/7)
+                            0.974927912181823607018131682993931217f,    // sin(4 pi/7)
+                            0.433883739117558120475768332848358754f};   // sin(6 pi/7)
+        const float2 x0 = v[0];
+        float2 p[3], m[3];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            p[t] = cadd(v[t + 1], v[6 - t]);
+            m[t] = csub(v[t + 1], v[6 - t]);
+        }
+        v[0] = make_float2(x0.x + (p[0].x + p[1].x + p[2].x), x0.y + (p[0].y + p[1].y + p[2].y));
+#pragma unroll
+        for (int k = 1; k <= 3; ++k) {
+            float2 a = x0, b = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int t = 1; t <= 3; ++t) {
+                const int e = (t * k) % 7;               // angle 2 pi e / 7
+                const int h = e <= 3 ? e : 7 - e;        // its cosine's index, and the sine's up to sign
+                const float ch = c[h - 1], sh = e <= 3 ? s[h - 1] : -s[h - 1];
+                a.x += ch * p[t - 1].x;
+                a.y += ch * p[t - 1].y;
+                b.x += sh * m[t - 1].x;
+                b.y += sh * m[t - 1].y;
+            }
+            const float2 r = mul_si<SIGN>(b);
+            v[k] = cadd(a, r);
+            v[7 - k] = csub(a, r);
+        }
+    }
+};
+
 // One Stockham autosort stage of radix R with current sub-transform size NS,
 // then the remaining stages.
 template <int N, int NS, int SIGN, int... Rs> struct Stages;
@@ -142,13 +181,17 @@ template <int N> struct Plan;
             Stages<N, 1, SIGN, __VA_ARGS__>::run(a, tw);                           \
         }                                                                          \
     };
+ER_FFT_PLAN(2, 2)
+ER_FFT_PLAN(3, 3)
 ER_FFT_PLAN(4, 4)
 ER_FFT_PLAN(5, 5)
 ER_FFT_PLAN(6, 2, 3)
+ER_FFT_PLAN(7, 7)
 ER_FFT_PLAN(8, 4, 2)
 ER_FFT_PLAN(9, 3, 3)
 ER_FFT_PLAN(10, 2, 5)
 ER_FFT_PLAN(12, 4, 3)
+ER_FFT_PLAN(15, 3, 5)
 ER_FFT_PLAN(16, 4, 4)
 ER_FFT_PLAN(18, 2, 3, 3)
 ER_FFT_PLAN(20, 4, 5)

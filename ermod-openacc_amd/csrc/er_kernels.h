@@ -598,6 +598,7 @@ __global__ void k_engfac_pppm(int K1, int K2, int K3, PPPMCoef pc, double i00, d
 // T layout: [chunk][H][K2][K3] (x3 fastest).
 // ---------------------------------------------------------------------------
 #define ER_SCH 8  // solute sites per LDS table chunk
+#define ER_DENSE_SITES 12  // most sites of the product form; above it the plane kernels spread + transform
 
 // offsets of the small-radix tables exp(+2 pi i k/r), r = 4..10, concatenated
 __host__ __device__ constexpr int tws_off(int r) { return r * (r - 1) / 2 - 6; }
@@ -1162,10 +1163,11 @@ __global__ void __launch_bounds__(RL * 16) k_pme_axis1_t(int nchunk, int K2, int
 }
 
 // ---------------------------------------------------------------------------
-// PME for grid shapes without a compiled plane or line kernel (any K, any
-// factors): the same two stages with direct DFTs, each output a sum over its
-// line with twiddles e^{+2 pi i k / K} from the tables, O(K) work per
-// element instead of O(log K).  The reference transforms any K1 x K2 x K3
+// PME for grid lengths with a prime factor above 7 (and, along axis 1, the
+// one-insertion launches of lengths without a compiled kernel): the same
+// two stages with direct DFTs, each output a sum over its line with twiddles
+// e^{+2 pi i k / K} from the tables, O(K) work per element instead of
+// O(log K).  The reference transforms any K1 x K2 x K3
 // (erdst/fft_iface.F90:38-50); these kernels keep that generality.
 // ---------------------------------------------------------------------------
 #define ER_GEN_NT 256
