@@ -695,6 +695,7 @@ extern "C" int er_create(const er_topology *topo, const er_params *prm, er_ctx *
     HIPCHK(c, upload_tw(c->d_tw3, c->K3, s));
     HIPCHK(c, upload_tw(c->d_twm, c->K1 / 2, s));
     for (int d = 0; d < 3; ++d) {
+        if (d == 0 ? fft_len_ok(c->K1) : plane_ok(c->K2, c->K3)) continue;  // compiled kernels
         std::vector<unsigned short> rev;
         if (!line_plan(prm->ms[d], c->lp[d], rev)) continue;
         HIPCHK(c, c->d_rev[d].ensure(rev.size()));
@@ -1664,14 +1665,22 @@ static void ecorr_slices(const er_ctx *c, int nch, int &kper, int &nks)
 
 // workgroups per insertion in the pair search: the slot's tuned value in a
 // batched run (the shape it was tuned for), else enough to fill the chip (at
-// least 4 per CU); a many-site solute reaches far, so its candidates are
-// spread over 16.  Every (insertion, molecule) sum has one owner whatever
-// the split, so the split never changes a result.
-static int pair_split(const Slot &sl, int nins, bool batched)
+// least 4 per CU, at most 64 per insertion and one per 128 molecules beyond
+// 16).  Solutes of more than 8 sites cost more per candidate and their
+// workgroups differ more: twice as many, and from 65 sites eight times, up to
+// 256 for a lone insertion.  Measured: a solution run's 150-site solute among
+// 12 000 waters 486 us in 16 workgroups, 41 us in 256; 256 insertions of it in
+// a 200 000-atom slab 1790 / 1390 / 1275 us in 4 / 16 / 32 each; 250
+// insertions of each of seven solutes of 2 to 45 sites 1072 / 686 / 691 / 868 us
+// in 1 / 4 / 8 / 16 each.  Every (insertion, molecule) sum has one owner
+// whatever the split, so the split never changes a result.
+static int pair_split(const er_ctx *c, const Slot &sl, int nins, bool batched)
 {
     if (batched && sl.pair_split > 0) return sl.pair_split;
-    if (sl.nslt > 8) return 16;
-    return std::max(1, std::min(16, (4 * 256 + nins - 1) / nins));
+    auto fill = [&](int blocks) { return (blocks + nins - 1) / nins; };
+    if (sl.nslt > 64) return std::max(8, std::min({256, fill(32 * 256), std::max(16, c->nummol / 32)}));
+    if (sl.nslt > 8) return std::max(4, std::min({256, fill(8 * 256), std::max(16, c->nummol / 32)}));
+    return std::max(1, std::min({64, fill(4 * 256), std::max(16, c->nummol / 128)}));
 }
 
 // The run's solutes end to end: the solutes of few sites first (dense plane
@@ -1699,7 +1708,7 @@ static int build_plan(er_ctx *c, const std::vector<int> &todo, int mode)
         d.ins_off = (int)ins;
         d.nins = nins;
         d.site_off = (int)site;
-        d.pair_split = pair_split(sl, batched ? nins : 1, batched);
+        d.pair_split = pair_split(c, sl, batched ? nins : 1, batched);
         d.pair_blk = (int)blk;
         ecorr_slices(c, nins, d.kper, d.nks);
         d.slice_off = z;

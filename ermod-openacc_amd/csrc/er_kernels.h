@@ -2429,78 +2429,22 @@ __device__ __forceinline__ float molecule_pair_sum_lds(const PairArgs &pa, const
     return e;
 }
 
-// The pair search and sums of one (insertion, part) block: solutes of at
-// most 8 sites take one thread per candidate molecule (k_pairs), larger ones
-// a group of lanes per molecule (k_pairs_many).  The two are separate kernels
-// so that each gets its own register allocation: the many-site kernel is
-// compiled for six waves per SIMD (the most its LDS allows), the few-site one
-// needs no such limit.  A launch covers the run's blocks of both classes;
-// each kernel returns at once from the other class's blocks.
-template <bool MANY>
-__device__ __forceinline__ void pairs_block(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
-    FrameConst fc, const int *__restrict__ molbeg, const uint4 *__restrict__ posu, const int *__restrict__ ljtype,
-    const float4 *__restrict__ molref, const float4 *__restrict__ segref, const float *__restrict__ rmolmax,
-    const unsigned int *__restrict__ cstart, const int *__restrict__ perm, const float4 *__restrict__ insposn_all,
-    const uint4 *__restrict__ insposu_all, const float4 *__restrict__ insref, const int *__restrict__ tag,
-    const float *__restrict__ ljene, const float *__restrict__ ljlensq, float *__restrict__ U)
+// Pair search, first half (both kernels): the candidate molecules of one
+// (insertion, part) block, handed to take(j, m) one by one with their bounding
+// spheres.  Part p of nsplit scans the cells c with c % nsplit == p.
+template <class TAKE>
+__device__ __forceinline__ void pair_candidates(const PairArgs &pa, const FrameConst &fc, const float4 &ref,
+                                                float cut, int part, int skipmol, float rmolmax,
+                                                const unsigned int *__restrict__ cstart,
+                                                const int *__restrict__ perm, const float4 *__restrict__ molref,
+                                                TAKE take)
 {
-    __shared__ int cand[ER_PAIR_CAP];
-    __shared__ int ncand, cnext;
-    __shared__ float4 sx[ER_PAIR_SCAP];
-    __shared__ uint4 sxu[ER_PAIR_SCAP];
-    __shared__ int stj[ER_PAIR_SCAP];
-    __shared__ float te[ER_PAIR_TCAP], ts[ER_PAIR_TCAP];
-    // workgroup b of the run (blk0 + blockIdx.x) belongs to the solute whose
-    // pair_blk range holds it; pair_split workgroups per insertion, part p
-    // owning the cells c with c % pair_split == p, so every (insertion,
-    // molecule) sum still has a single owner
-    const int b = blk0 + blockIdx.x;
-    const int ks = slot_find(nslot, b, [&](int m) { return sd[m].pair_blk; });
-    PairArgs pa = pa0;
-    pa.nsplit = sd[ks].pair_split;
-    pa.nslt = sd[ks].nslt;
-    if ((pa.nslt > 8) != MANY) return;  // the other kernel's block
-    const int bl = b - sd[ks].pair_blk;
-    const int nl = bl / pa.nsplit, part = bl % pa.nsplit;
-    const int n = sd[ks].ins_off + nl;
-    const __attribute__((address_space(1))) int *sltlj = gptr(sd[ks].sltlj);
-    // the insertion's sites (molecule_pair_sum reads them as insertion 0)
-    const float4 *__restrict__ insposn = insposn_all + sd[ks].site_off + (size_t)nl * pa.nslt;
-    const uint4 *__restrict__ insposu = insposu_all + sd[ks].site_off + (size_t)nl * pa.nslt;
     const int tid = threadIdx.x, NT = blockDim.x;
-    const float4 ref = insref[n];
-    const float cut = fmaxf(pa.pp.upljcut, pa.pp.elecut) + ref.w + 1e-3f;
-    const bool soln = tag != nullptr;
-    const int skipmol = soln ? tag[n] : -1;
-    const int slt_a0 = soln ? molbeg[skipmol] : 0;
-    const size_t urow = ((size_t)(n / pa.NI) * pa.nmol) * pa.NI + (n % pa.NI);
-    // the insertion's sites and the LJ tables in LDS when they fit
-    const int nt2 = pa.ntype * pa.ntype;
-    const bool in_lds = pa.nslt <= ER_PAIR_SCAP && nt2 <= ER_PAIR_TCAP;
-    if (tid == 0) ncand = 0;
-    if (tid == 0) cnext = 0;  // many-site path: the next candidate a wave takes
-    if (in_lds) {
-        for (int k = tid; k < pa.nslt; k += NT) {
-            sx[k] = insposn[k];
-            sxu[k] = insposu[k];
-            stj[k] = soln ? ljtype[slt_a0 + k] : sltlj[k];
-        }
-        for (int k = tid; k < nt2; k += NT) {
-            te[k] = ljene[k];
-            ts[k] = ljlensq[k];
-        }
-    }
-    __syncthreads();
-    auto pair_sum = [&](int j) {
-        return in_lds ? molecule_pair_sum_lds(pa, fc, j, molbeg, posu, ljtype, sxu, stj, te, ts)
-                      : molecule_pair_sum(pa, fc, 0, j, molbeg, posu, ljtype, insposu, sltlj, slt_a0, soln, ljene,
-                                          ljlensq);
-    };
     int cx, cy, cz;
     site_cell(fc, ref.x, ref.y, ref.z, pa.nc, cx, cy, cz);
     // a molecule centre within distance d of the search centre lies at most
     // ceil(d / width) cells away along every axis
-    const int nreach = (int)ceilf((cut + rmolmax[0]) / pa.cell_w);
+    const int nreach = (int)ceilf((cut + rmolmax) / pa.cell_w);
     const int span = min(2 * nreach + 1, pa.nc);  // distinct cells per axis
     const int lo = (span == pa.nc) ? 0 : -nreach;
     const int ncell = span * span * span;
@@ -2527,95 +2471,15 @@ __device__ __forceinline__ void pairs_block(PairArgs pa0, int blk0, int nslot, c
                 float ddx = m.x - ref.x, ddy = m.y - ref.y, ddz = m.z - ref.z;
                 min_image(fc, ddx, ddy, ddz);
                 const float lim = cut + m.w;
-                if (ddx * ddx + ddy * ddy + ddz * ddz <= lim * lim) {
-                    const int slot = atomicAdd(&ncand, 1);
-                    if (slot < ER_PAIR_CAP) cand[slot] = j;
-                    else  // list full: evaluate in place (same arithmetic, same single owner)
-                        U[urow + (size_t)j * pa.NI] += pair_sum(j);
-                }
+                if (ddx * ddx + ddy * ddy + ddz * ddz <= lim * lim) take(j);
             }
         }
-    }
-    __syncthreads();
-    const int nc = min(ncand, ER_PAIR_CAP);
-    if constexpr (!MANY) {  // few sites: one thread per candidate molecule
-        for (int c = tid; c < nc; c += NT) {
-            const int jm = cand[c];
-            U[urow + (size_t)jm * pa.NI] += pair_sum(jm);
-        }
-        return;
-    }
-    // many sites: a group of GS lanes (16, 32 or 64) per candidate molecule;
-    // lane g sums the sites g, g + GS, ... over the molecule's atoms (atom
-    // order), then a fixed xor tree adds the lanes (deterministic)
-    const int GS = pa.nslt <= 16 ? 16 : (pa.nslt <= 32 ? 32 : 64);
-    const int cpw = 64 / GS, lane = tid & 63;
-    const int grp = lane / GS, gl = lane % GS;
-    const float skip2 = pair_skip2(pa.pp);
-    const float skipc = fmaxf(pa.pp.upljcut, pa.pp.elecut) * 1.0001f + 1e-3f;
-    auto site_sum = [&](int s, int jm) {
-        const float4 xa = in_lds ? sx[s] : insposn[s];
-        const uint4 xu = in_lds ? sxu[s] : insposu[s];
-        const int ti = in_lds ? stj[s] : (soln ? ljtype[slt_a0 + s] : sltlj[s]);
-        float e = 0.0f;
-        // the molecule's centre and reach radius: beyond cutoff + reach,
-        // every site pair is beyond both cutoffs (triangle inequality
-        // on minimum images), so the site's sum is +0
-        const float4 m = molref[jm];
-        float rx = xa.x - m.x, ry = xa.y - m.y, rz = xa.z - m.z;
-        min_image(fc, rx, ry, rz);
-        const float lim = skipc + m.w;
-        if (rx * rx + ry * ry + rz * rz > lim * lim) return e;
-        // a molecule of three or more segments: the same test per segment,
-        // whose skipped pairs all fail the per-pair test below (same sum,
-        // same order)
-        const int b0 = molbeg[jm], b1 = molbeg[jm + 1];
-        const bool segmented = b1 - b0 > 2 * ER_SEG;
-        for (int s0 = b0; s0 < b1; s0 += ER_SEG) {
-            if (segmented) {
-                const float4 q = segref[s0];
-                float qx = xa.x - q.x, qy = xa.y - q.y, qz = xa.z - q.z;
-                min_image(fc, qx, qy, qz);
-                const float ql = skipc + q.w;
-                if (qx * qx + qy * qy + qz * qz > ql * ql) continue;
-            }
-            for (int b = s0; b < min(s0 + ER_SEG, b1); ++b) {
-                const uint4 xb = posu[b];
-                const int tj = ljtype[b];
-                const float d2 = lattice_d2(fc, xu, xb);
-                if (d2 > skip2) continue;
-                const float le = in_lds ? te[ti + pa.ntype * tj] : ljene[ti + pa.ntype * tj];
-                const float ls = in_lds ? ts[ti + pa.ntype * tj] : ljlensq[ti + pa.ntype * tj];
-                e += pair_energy(pa.pp, d2, xa.w, __uint_as_float(xb.w), le, ls);
-            }
-        }
-        return e;
-    };
-    // a wave takes its next cpw candidates from a shared counter when it is
-    // done with the last ones (molecules of very different sizes balance
-    // across the waves); each candidate's sum is still one group's, in the
-    // same order, so the results do not depend on which wave takes it
-    int c0;
-    {
-        int take = 0;
-        if (lane == 0) take = atomicAdd(&cnext, cpw);
-        c0 = __shfl(take, 0, 64);
-    }
-    while (c0 < nc) {  // wave-uniform
-        const int c = c0 + grp;
-        const bool live = c < nc;
-        const int jm = live ? cand[c] : 0;
-        float e = 0.0f;
-        if (live)
-            for (int st = gl; st < pa.nslt; st += GS) e += site_sum(st, jm);
-        for (int off = GS / 2; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
-        if (live && gl == 0) U[urow + (size_t)jm * pa.NI] += e;
-        int take = 0;
-        if (lane == 0) take = atomicAdd(&cnext, cpw);
-        c0 = __shfl(take, 0, 64);
     }
 }
 
+// Pairs of the solutes of at most 8 sites, one (insertion, part) block per
+// workgroup: one thread per candidate molecule.  A launch covers the run's
+// blocks of both classes; each kernel returns at once from the other's.
 __global__ void __launch_bounds__(256) k_pairs(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
     FrameConst fc, const int *__restrict__ molbeg, const uint4 *__restrict__ posu, const int *__restrict__ ljtype,
     const float4 *__restrict__ molref, const float4 *__restrict__ segref, const float *__restrict__ rmolmax,
@@ -2623,11 +2487,100 @@ __global__ void __launch_bounds__(256) k_pairs(PairArgs pa0, int blk0, int nslot
     const uint4 *__restrict__ insposu_all, const float4 *__restrict__ insref, const int *__restrict__ tag,
     const float *__restrict__ ljene, const float *__restrict__ ljlensq, float *__restrict__ U)
 {
-    pairs_block<false>(pa0, blk0, nslot, sd, fc, molbeg, posu, ljtype, molref, segref, rmolmax, cstart, perm,
-                       insposn_all, insposu_all, insref, tag, ljene, ljlensq, U);
+    __shared__ int cand[ER_PAIR_CAP];
+    __shared__ int ncand;
+    __shared__ uint4 sxu[8];
+    __shared__ int stj[8];
+    __shared__ float te[ER_PAIR_TCAP], ts[ER_PAIR_TCAP];
+    // workgroup b of the run (blk0 + blockIdx.x) belongs to the solute whose
+    // pair_blk range holds it; pair_split workgroups per insertion, part p
+    // owning the cells c with c % pair_split == p, so every (insertion,
+    // molecule) sum still has a single owner
+    const int b = blk0 + blockIdx.x;
+    const int ks = slot_find(nslot, b, [&](int m) { return sd[m].pair_blk; });
+    PairArgs pa = pa0;
+    pa.nsplit = sd[ks].pair_split;
+    pa.nslt = sd[ks].nslt;
+    if (pa.nslt > 8) return;  // the other kernel's block
+    const int bl = b - sd[ks].pair_blk;
+    const int nl = bl / pa.nsplit, part = bl % pa.nsplit;
+    const int n = sd[ks].ins_off + nl;
+    const __attribute__((address_space(1))) int *sltlj = gptr(sd[ks].sltlj);
+    // the insertion's sites (molecule_pair_sum reads them as insertion 0)
+    const uint4 *__restrict__ insposu = insposu_all + sd[ks].site_off + (size_t)nl * pa.nslt;
+    const int tid = threadIdx.x, NT = blockDim.x;
+    const float4 ref = insref[n];
+    const float cut = fmaxf(pa.pp.upljcut, pa.pp.elecut) + ref.w + 1e-3f;
+    const bool soln = tag != nullptr;
+    const int skipmol = soln ? tag[n] : -1;
+    const int slt_a0 = soln ? molbeg[skipmol] : 0;
+    const size_t urow = ((size_t)(n / pa.NI) * pa.nmol) * pa.NI + (n % pa.NI);
+    // the insertion's sites and the LJ tables in LDS when they fit
+    const int nt2 = pa.ntype * pa.ntype;
+    const bool in_lds = nt2 <= ER_PAIR_TCAP;
+    if (tid == 0) ncand = 0;
+    if (in_lds) {
+        if (tid < pa.nslt) {
+            sxu[tid] = insposu[tid];
+            stj[tid] = soln ? ljtype[slt_a0 + tid] : sltlj[tid];
+        }
+        for (int k = tid; k < nt2; k += NT) {
+            te[k] = ljene[k];
+            ts[k] = ljlensq[k];
+        }
+    }
+    __syncthreads();
+    auto pair_sum = [&](int j) __attribute__((always_inline)) {
+        return in_lds ? molecule_pair_sum_lds(pa, fc, j, molbeg, posu, ljtype, sxu, stj, te, ts)
+                      : molecule_pair_sum(pa, fc, 0, j, molbeg, posu, ljtype, insposu, sltlj, slt_a0, soln, ljene,
+                                          ljlensq);
+    };
+    pair_candidates(pa, fc, ref, cut, part, skipmol, rmolmax[0], cstart, perm, molref, [&](int j) __attribute__((always_inline)) {
+        const int slot = atomicAdd(&ncand, 1);
+        if (slot < ER_PAIR_CAP) cand[slot] = j;
+        else  // list full: evaluate in place (same arithmetic, same single owner)
+            U[urow + (size_t)j * pa.NI] += pair_sum(j);
+    });
+    __syncthreads();
+    const int nc = min(ncand, ER_PAIR_CAP);
+    for (int c = tid; c < nc; c += NT) {
+        const int jm = cand[c];
+        U[urow + (size_t)jm * pa.NI] += pair_sum(jm);
+    }
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
+// row_shl:R, lane i of a 16-lane DPP row reads lane i + R (0 past the row)
+template <int R>
+__device__ __forceinline__ float row_shl(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x100 + R, 0xf, 0xf, true));
+}
+
+#define ER_PM_CLU 32                  // clusters of 8 sites with a bounding sphere (ER_PAIR_SCAP sites)
+#define ER_PM_ATOMS (2 * ER_SEG)      // molecules of more atoms go segment by segment
+#define ER_PM_SUMS 512                // site sums per wave
+
+// Pairs of the solutes of more than 8 sites.  The sum of a (site, molecule)
+// runs over the molecule's atoms in order, the site sums are added over the
+// sites g, g + 64, ... of lane class g and then in a fixed tree: work is laid
+// on the lanes so that those orders hold by themselves.
+//  - Molecules of up to 16 atoms, up to 32 per wave: the (site, molecule)
+//    pairs whose site reaches the molecule are listed first, so that full
+//    waves of them run over the molecules' atoms; each leaves its site sum in
+//    LDS for the tree.
+//  - Larger molecules, one per wave, segment by segment: lane (i, b)
+//    forms the pair (site i of a cluster, atom b of the segment), and the
+//    segment's eight terms of a site are added in atom order with row
+//    shifts.  A segment meets only the clusters whose bounding sphere its own
+//    reaches (one ballot over the clusters).
+// Skipped pairs lie beyond both cutoffs (triangle inequality on minimum
+// images, with a margin over FP32 rounding) and would add +0.
+// Bound by VALU and the LJ-table gathers of the pairs in reach.  A lane per
+// site looping over the atoms (the earlier form) left most lanes idle: 256
+// insertions of a 150-site solute among 200 000 atoms took 2112 us there, 1280 us
+// here; 250 insertions each of 9 to 45 sites among waters and 9-site molecules 800
+// and 545 us.
+__global__ void __launch_bounds__(256)
 k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
     FrameConst fc, const int *__restrict__ molbeg, const uint4 *__restrict__ posu, const int *__restrict__ ljtype,
     const float4 *__restrict__ molref, const float4 *__restrict__ segref, const float *__restrict__ rmolmax,
@@ -2635,8 +2588,200 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
     const uint4 *__restrict__ insposu_all, const float4 *__restrict__ insref, const int *__restrict__ tag,
     const float *__restrict__ ljene, const float *__restrict__ ljlensq, float *__restrict__ U)
 {
-    pairs_block<true>(pa0, blk0, nslot, sd, fc, molbeg, posu, ljtype, molref, segref, rmolmax, cstart, perm,
-                      insposn_all, insposu_all, insref, tag, ljene, ljlensq, U);
+    __shared__ int cand[ER_PAIR_CAP];  // small molecules from the front, large ones from the back
+    __shared__ int ncand, nsmall, nlarge, nextS, nextL;
+    __shared__ float4 sx[ER_PAIR_SCAP];
+    __shared__ uint4 sxu[ER_PAIR_SCAP];
+    __shared__ int stj[ER_PAIR_SCAP];
+    __shared__ float sums[4][ER_PM_SUMS];  // per wave: site sums of its molecules
+    __shared__ unsigned short list[4][ER_PM_SUMS];
+    __shared__ float4 clu[ER_PM_CLU];
+    const int b = blk0 + blockIdx.x;  // as in k_pairs
+    const int ks = slot_find(nslot, b, [&](int m) { return sd[m].pair_blk; });
+    PairArgs pa = pa0;
+    pa.nsplit = sd[ks].pair_split;
+    pa.nslt = sd[ks].nslt;
+    if (pa.nslt <= 8) return;  // the other kernel's block
+    const int bl = b - sd[ks].pair_blk;
+    const int nl = bl / pa.nsplit, part = bl % pa.nsplit;
+    const int n = sd[ks].ins_off + nl;
+    const __attribute__((address_space(1))) int *sltlj = gptr(sd[ks].sltlj);
+    const float4 *__restrict__ insposn = insposn_all + sd[ks].site_off + (size_t)nl * pa.nslt;
+    const uint4 *__restrict__ insposu = insposu_all + sd[ks].site_off + (size_t)nl * pa.nslt;
+    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const float4 ref = insref[n];
+    const float cut = fmaxf(pa.pp.upljcut, pa.pp.elecut) + ref.w + 1e-3f;
+    const bool soln = tag != nullptr;
+    const int skipmol = soln ? tag[n] : -1;
+    const int slt_a0 = soln ? molbeg[skipmol] : 0;
+    const size_t urow = ((size_t)(n / pa.NI) * pa.nmol) * pa.NI + (n % pa.NI);
+    const bool in_lds = pa.nslt <= ER_PAIR_SCAP;  // the sites
+    if (tid == 0) ncand = nsmall = nlarge = nextS = nextL = 0;
+    if (in_lds)
+        for (int k = tid; k < pa.nslt; k += NT) {
+            sx[k] = insposn[k];
+            sxu[k] = insposu[k];
+            stj[k] = soln ? ljtype[slt_a0 + k] : sltlj[k];
+        }
+    __syncthreads();
+    const int nclu = (pa.nslt + 7) >> 3;
+    if (in_lds && tid < nclu) clu[tid] = atom_sphere(fc, sx, tid * 8, min(tid * 8 + 8, pa.nslt));
+    pair_candidates(pa, fc, ref, cut, part, skipmol, rmolmax[0], cstart, perm, molref, [&](int j) __attribute__((always_inline)) {
+        if (atomicAdd(&ncand, 1) < ER_PAIR_CAP) {
+            if (molbeg[j + 1] - molbeg[j] <= ER_PM_ATOMS) cand[atomicAdd(&nsmall, 1)] = j;
+            else cand[ER_PAIR_CAP - 1 - atomicAdd(&nlarge, 1)] = j;
+        } else {  // list full: evaluate in place, same single owner
+            U[urow + (size_t)j * pa.NI] += molecule_pair_sum(pa, fc, 0, j, molbeg, posu, ljtype, insposu, sltlj,
+                                                              slt_a0, soln, ljene, ljlensq);
+        }
+    });
+    __syncthreads();
+    const int ns = nsmall, nlg = nlarge;
+    const float skip2 = pair_skip2(pa.pp);
+    const float skipc = fmaxf(pa.pp.upljcut, pa.pp.elecut) * 1.0001f + 1e-3f;
+    const int i8 = lane >> 3, w8 = lane & 7;
+    auto site_u = [&](int s) { return in_lds ? sxu[s] : insposu[s]; };
+    auto site_t = [&](int s) { return in_lds ? stj[s] : (soln ? ljtype[slt_a0 + s] : sltlj[s]); };
+    // a wave takes its next molecules from a shared counter when it is done
+    // with the last ones; each sum is one wave's, in the same order, whichever
+    // wave takes it
+    auto next = [&](int *ctr, int k) {
+        int take = 0;
+        if (lane == 0) take = atomicAdd(ctr, k);
+        return __builtin_amdgcn_readfirstlane(take);
+    };
+    for (int c = next(&nextL, 1); c < nlg; c = next(&nextL, 1)) {
+        const int jm = __builtin_amdgcn_readfirstlane(cand[ER_PAIR_CAP - 1 - c]);
+        const int b0 = molbeg[jm], b1 = molbeg[jm + 1];
+        float e = 0.0f;
+        for (int sb = 0; sb < pa.nslt; sb += ER_PAIR_SCAP) {  // 256 sites at a time (one block of them in LDS)
+            const int se = min(pa.nslt, sb + ER_PAIR_SCAP);
+            for (int st = lane; st < se - sb; st += 64) sums[wv][st] = 0.0f;
+            for (int s0 = b0; s0 < b1; s0 += ER_SEG) {
+                const int at = min(s0 + w8, b1 - 1);
+                const bool atom = s0 + w8 < b1;
+                const uint4 xb = posu[at];
+                const int tj = ljtype[at];
+                unsigned long long todo = ~0ull >> (64 - ((se - sb + 7) >> 3));  // at most 32 clusters
+                if (in_lds) {
+                    const float4 q = segref[s0], k = clu[min(lane, nclu - 1)];
+                    float qx = k.x - q.x, qy = k.y - q.y, qz = k.z - q.z;
+                    min_image(fc, qx, qy, qz);
+                    const float ql = skipc + q.w + k.w;
+                    todo &= __ballot(!(qx * qx + qy * qy + qz * qz > ql * ql));
+                }
+                while (todo) {
+                    const int cl = __builtin_ctzll(todo);
+                    todo &= todo - 1;
+                    const int s = sb + cl * 8 + i8, sc = min(s, pa.nslt - 1);
+                    const uint4 xu = site_u(sc);
+                    const float d2 = lattice_d2(fc, xu, xb);
+                    const bool act = s < se && atom && !(d2 > skip2);
+                    if (!__ballot(act)) continue;
+                    float t = 0.0f;
+                    if (act) {
+                        const int ti = site_t(sc);
+                        t = pair_energy(pa.pp, d2, __uint_as_float(xu.w), __uint_as_float(xb.w),
+                                        ljene[ti + pa.ntype * tj], ljlensq[ti + pa.ntype * tj]);
+                    }
+                    // lanes b = 0 hold the site's sum: its atoms in order
+                    float es = sums[wv][sc - sb];
+                    es += t;
+                    es += row_shl<1>(t);
+                    es += row_shl<2>(t);
+                    es += row_shl<3>(t);
+                    es += row_shl<4>(t);
+                    es += row_shl<5>(t);
+                    es += row_shl<6>(t);
+                    es += row_shl<7>(t);
+                    if (w8 == 0 && s < se) sums[wv][s - sb] = es;
+                }
+            }
+            for (int st = lane; st < se - sb; st += 64) e += sums[wv][st];
+        }
+        for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
+        if (lane == 0) U[urow + (size_t)jm * pa.NI] += e;
+    }
+    // molecules per batch: as many as the site sums of one fit in the wave's share
+    // (fewer sites, more molecules: the list has to fill whole waves)
+    const int wsh = pa.nslt > 256 ? 0 : 31 - __clz(ER_PM_SUMS / pa.nslt), W = 1 << wsh;
+    const int GS = pa.nslt <= 16 ? 16 : (pa.nslt <= 32 ? 32 : 64);  // lane classes of the final tree
+    for (int c0 = next(&nextS, W); c0 < ns; c0 = next(&nextS, W)) {
+        const int w = lane & (W - 1);  // this lane's molecule of the batch
+        const bool live = c0 + w < ns;
+        const int jw = cand[live ? c0 + w : c0];
+        const float4 m = molref[jw];
+        const int bw0 = molbeg[jw], bw1 = molbeg[jw + 1];
+        const float lim = skipc + m.w;
+        float e1 = 0.0f;  // W = 1: the lane class's sum so far
+        for (int sb = 0; sb < pa.nslt; sb += ER_PM_SUMS) {
+            const int nsb = min(ER_PM_SUMS, pa.nslt - sb), nit = nsb << wsh;
+            // molecules of up to four atoms from the front of the list, longer
+            // ones from its back: a wave's lanes run about as many atoms
+            int nf = 0, nbk = 0;
+            for (int i0 = 0; i0 < nit; i0 += 64) {
+                const int s = min((i0 + lane) >> wsh, nsb - 1);
+                const float4 xa = in_lds ? sx[s] : insposn[sb + s];
+                // beyond cutoff + reach of the molecule's centre every pair of
+                // this site is beyond both cutoffs
+                float rx = xa.x - m.x, ry = xa.y - m.y, rz = xa.z - m.z;
+                min_image(fc, rx, ry, rz);
+                const bool in = i0 + lane < nit;
+                const bool near = live && in && !(rx * rx + ry * ry + rz * rz > lim * lim);
+                const unsigned long long below = (1ull << lane) - 1ull;
+                const unsigned long long mf = __ballot(near && bw1 - bw0 <= 4), mb = __ballot(near && bw1 - bw0 > 4);
+                if (near)
+                    list[wv][bw1 - bw0 <= 4 ? nf + __popcll(mf & below) : ER_PM_SUMS - 1 - nbk - __popcll(mb & below)] =
+                        (unsigned short)(s << 6 | w);
+                if (in) sums[wv][w * nsb + s] = 0.0f;
+                nf += __popcll(mf);
+                nbk += __popcll(mb);
+            }
+            const int nfw = (nf + 63) & ~63, nlist = nfw + nbk;  // whole waves of either kind
+            for (int l0 = 0; l0 < nlist; l0 += 64) {
+                const bool front = l0 < nfw;
+                const int l = (front ? l0 : l0 - nfw) + lane;
+                const bool on = l < (front ? nf : nbk);
+                const int ent = list[wv][!on ? (front ? 0 : ER_PM_SUMS - 1) : front ? l : ER_PM_SUMS - 1 - l];
+                const int s = ent >> 6, we = ent & 63;
+                const int b0 = __shfl(bw0, we, 64), b1 = __shfl(bw1, we, 64);
+                const uint4 xu = site_u(sb + s);
+                const int ti = site_t(sb + s);
+                float e = 0.0f;
+                if (on)
+                    for (int bb = b0; bb < b1; bb += 4) {  // atoms in order, four loads in flight
+                        uint4 xb[4];
+                        int tb[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const int at = min(bb + k, b1 - 1);
+                            xb[k] = posu[at];
+                            tb[k] = ljtype[at];
+                        }
+                        for (int k = 0; k < 4; ++k) {
+                            const uint4 x = k == 0 ? xb[0] : k == 1 ? xb[1] : k == 2 ? xb[2] : xb[3];
+                            const int tj = k == 0 ? tb[0] : k == 1 ? tb[1] : k == 2 ? tb[2] : tb[3];
+                            const float d2 = lattice_d2(fc, xu, x);
+                            if (bb + k < b1 && !(d2 > skip2))
+                                e += pair_energy(pa.pp, d2, __uint_as_float(xu.w), __uint_as_float(x.w),
+                                                 ljene[ti + pa.ntype * tj], ljlensq[ti + pa.ntype * tj]);
+                        }
+                    }
+                if (on) sums[wv][we * nsb + s] = e;
+            }
+            // the site sums of lane class g, added over g, g + GS, ...
+            const int grp = lane / GS, gl = lane % GS;
+            for (int w0 = 0; w0 < W; w0 += 64 / GS) {
+                float e = e1;
+                for (int st = gl; st < nsb; st += GS) e += sums[wv][(w0 + grp) * nsb + st];
+                if (W == 1) e1 = e;
+                if (sb + nsb < pa.nslt) continue;  // W = 1: more sites to come
+                for (int off = GS / 2; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
+                if (gl == 0 && c0 + w0 + grp < ns) U[urow + (size_t)cand[c0 + w0 + grp] * pa.NI] += e;
+            }
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
