@@ -128,6 +128,7 @@ struct er_ctx {
     std::vector<int> molbeg;       // 0-based [nummol+1]
     std::vector<int> uvspec;       // [nummol]
     std::vector<float> molq;       // [nummol]
+    int maxmol = 1;                // atoms of the largest molecule
     std::vector<int> sp_begin, sp_end;
     float qtot = 0.f;              // sum of physical molecule charges
 
@@ -597,6 +598,7 @@ extern "C" int er_create(const er_topology *topo, const er_params *prm, er_ctx *
         return bad(fail(c, ER_E_ARG, "er_create: mol_begin_index inconsistent with numatm"));
     for (int j = 0; j < c->nummol; ++j)
         if (c->molbeg[j + 1] <= c->molbeg[j]) return bad(fail(c, ER_E_ARG, "er_create: empty molecule"));
+    for (int j = 0; j < c->nummol; ++j) c->maxmol = std::max(c->maxmol, c->molbeg[j + 1] - c->molbeg[j]);
     std::vector<int> lj(c->numatm);
     for (int a = 0; a < c->numatm; ++a) {
         lj[a] = topo->ljtype[a] - 1;
@@ -934,13 +936,6 @@ extern "C" int er_set_solute_molecules(er_ctx *c, int32_t nslt, const int32_t *t
 
 // Morton keys of nc cells per axis: coordinates below the next power of two
 // p interleave into keys below p^3 (32^3 at most)
-static int morton_keys(int nc)
-{
-    int p = 1;
-    while (p < nc) p <<= 1;
-    return p * p * p;
-}
-
 // realcal_prepare's cell handling (realcal.F90:776-896) + get_inverted_cell
 static int frame_cell(er_ctx *c, const float *cell)
 {
@@ -1106,7 +1101,7 @@ static int frame_cell(er_ctx *c, const float *cell)
         }
         c->cell_wmin = wmin;
         c->nc = std::max(1, std::min(32, (int)(wmin / (c->cell_min > 0.f ? c->cell_min : 3.5f))));
-        c->ncell = morton_keys(c->nc);
+        c->ncell = cell_keys(c->nc);
         c->cell_w = (float)(wmin / c->nc);
     }
     c->cell_changed = !c->have_prev_cell || std::memcmp(c->prev_cell, cell, sizeof c->prev_cell) != 0;
@@ -1552,6 +1547,22 @@ static hipError_t join_atoms(er_ctx *c)
     return hipStreamWaitEvent(c->stream, c->ev_atoms, 0);
 }
 
+// f(integral_constant) of the spline order (0: no reciprocal part)
+template <class F> static void with_order(int ord, F f)
+{
+    switch (ord) {
+    case 0: f(std::integral_constant<int, 0>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 7: f(std::integral_constant<int, 7>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 9: f(std::integral_constant<int, 9>{}); break;
+    case 10: f(std::integral_constant<int, 10>{}); break;
+    }
+}
+
 static hipError_t prep_frame(er_ctx *c)
 {
     const int B = 256;
@@ -1587,22 +1598,42 @@ static hipError_t prep_frame(er_ctx *c)
             HIPCHK_E(hipEventRecord(c->ev_in, c->stream));
             HIPCHK_E(hipStreamWaitEvent(s2, c->ev_in, 0));
         }
-        // five launches: atoms (and the counters cleared), molecules, both
-        // counting passes, both scans, then the brick records with the
-        // molecules' scatter into cell order
-        hipLaunchKernelGGL(k_prep_atoms, dim3((c->numatm + B - 1) / B), dim3(B), 0, s2, c->numatm, c->d_sitepos,
-                           c->d_charge.p, c->fc, c->K1, c->K2, c->K3, c->ord, c->d_posn.p, c->d_posu.p, c->d_splw.p,
-                           c->d_splg.p, c->d_ccnt.p, c->ncell, c->d_bcnt.p, c->nbrick, c->d_rmolmax.p);
-        hipLaunchKernelGGL(k_prep_mols, dim3((c->nummol + B - 1) / B), dim3(B), 0, s2, c->nummol,
-                           c->d_molbeg.p, c->d_posn.p, c->fc, c->d_molref.p, c->d_rmolmax.p, c->d_segref.p);
+        // atoms and molecule spheres (and the counters cleared), both sorts'
+        // counts and scans (one launch for small frames), then the brick
+        // records with the molecules' scatter into cell order.  Bare Coulomb
+        // has no grid: no splines, no bricks.
+        const bool bare = c->prm.cltype == 0;
+        const int nbrick = bare ? 0 : c->nbrick;
+        int gsh = 0;  // lanes per molecule: one up to four atoms, then about four atoms a lane
+        while (gsh < 4 && (4 << gsh) < c->maxmol) ++gsh;
+        const int nab = (c->numatm + B - 1) / B;
+        const long mthreads = (long)c->nummol << gsh;
+        const dim3 grid((unsigned)(nab + (mthreads + B - 1) / B));
+        auto prep = [&](auto ord) {
+            hipLaunchKernelGGL(k_prep_frame<decltype(ord)::value>, grid, dim3(B), 0, s2, c->numatm, nab, c->d_sitepos,
+                               c->d_charge.p, c->fc, c->K1, c->K2, c->K3, c->d_posn.p, c->d_posu.p, c->d_splw.p,
+                               c->d_splg.p, c->d_ccnt.p, c->ncell, c->d_bcnt.p, nbrick, c->d_rmolmax.p, c->nummol,
+                               gsh, c->d_molbeg.p, c->d_molref.p, c->d_segref.p);
+        };
+        with_order(bare ? 0 : c->ord, prep);
         // spatial order of the molecules (the cell list) and of the atoms by PME brick
         const int nsort = c->nummol + c->numatm;
-        hipLaunchKernelGGL(k_sort_count, dim3((nsort + B - 1) / B), dim3(B), 0, s2, c->nummol, c->d_molref.p,
-                           c->fc, c->nc, c->d_ccnt.p, c->d_keyrank.p, c->numatm, c->d_splg.p, c->K1, c->K2, c->K3,
-                           c->nbx, c->nby, brick_z(c->ord), c->d_bcnt.p, c->d_akeyrank.p);
-        hipLaunchKernelGGL(k_sort_scan, dim3(2), dim3(1024), 0, s2, c->ncell, c->d_ccnt.p, c->d_cstart.p, c->nbrick,
-                           c->d_bcnt.p, c->d_bstart.p);
-        switch (c->ord) {
+        const SortGrid sg{c->nc, c->K1, c->K2, c->K3, c->nbx, c->nby, brick_z(c->ord), nbrick};
+        if (nsort <= ER_SORT_ITEMS && c->ncell + nbrick <= ER_SORT_LDS) {
+            hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(1024), (c->ncell + nbrick) * sizeof(unsigned int), s2,
+                               c->nummol, c->d_molref.p, c->fc, sg, c->ncell, c->d_cstart.p, c->d_keyrank.p,
+                               c->d_rmolmax.p, c->numatm, c->d_splg.p, c->d_bstart.p, c->d_akeyrank.p);
+        } else {
+            const int nmb = (c->nummol + 1023) / 1024, per = 1024 * ER_SORT_APT;
+            const int nbb = nbrick ? (c->numatm + per - 1) / per : 0;
+            const size_t lds = nbrick <= ER_SORT_LDS ? nbrick * sizeof(unsigned int) : 0;
+            hipLaunchKernelGGL(k_sort_count, dim3(nmb + nbb), dim3(1024), lds, s2, c->nummol, nmb, c->d_molref.p,
+                               c->fc, sg, c->d_ccnt.p, c->d_keyrank.p, c->d_rmolmax.p, c->numatm, c->d_splg.p,
+                               c->d_bcnt.p, c->d_akeyrank.p);
+            hipLaunchKernelGGL(k_sort_scan, dim3(nbrick ? 2 : 1), dim3(256), 0, s2, c->ncell, c->d_ccnt.p,
+                               c->d_cstart.p, nbrick, c->d_bcnt.p, c->d_bstart.p);
+        }
+        switch (bare ? 0 : c->ord) {
 #define ER_BREC(O)                                                                                              \
     case O:                                                                                                     \
         hipLaunchKernelGGL(k_brick_records<O>, dim3((nsort + B - 1) / B), dim3(B), 0, s2, c->numatm,            \
@@ -1612,7 +1643,7 @@ static hipError_t prep_frame(er_ctx *c)
         break;
             ER_BREC(3) ER_BREC(4) ER_BREC(5) ER_BREC(6) ER_BREC(7) ER_BREC(8)
 #undef ER_BREC
-        default:  // orders 9 and 10: the per-molecule gather, no records
+        default:  // orders 9 and 10 (the per-molecule gather) and bare Coulomb: no records
             hipLaunchKernelGGL(k_cell_scatter, dim3((c->nummol + B - 1) / B), dim3(B), 0, s2, c->nummol,
                                c->d_keyrank.p, c->d_cstart.p, c->d_perm.p);
             break;
@@ -2062,39 +2093,44 @@ static int run_slots(er_ctx *c, const std::vector<int> &todo, int mode)
     {
         ProfScope ps(c, ER_K_PREP);
         HIPCHK(c, prep_frame(c));
-        if (!soln)  // the insertions' coordinates, solutes end to end
+        const bool bare = c->prm.cltype == 0;
+        InsSource src{};
+        int maxslt = 0;
+        if (!soln) {
+            if (nslot > ER_INS_PTRS) src.cat = c->d_sltcat.p;  // the insertions' coordinates, solutes end to end
             for (int i = 0; i < nslot; ++i) {
                 const Slot &sl = c->slots[P.order[i]];
-                const size_t n = (size_t)P.desc[i].nins * sl.nslt * 3;
-                HIPCHK(c, hipMemcpyAsync(c->d_sltcat.p + (size_t)P.desc[i].site_off * 3, sl.d_sltpos,
-                                         n * sizeof(float), hipMemcpyDeviceToDevice, c->stream));
+                if (src.cat)
+                    HIPCHK(c, hipMemcpyAsync(c->d_sltcat.p + (size_t)P.desc[i].site_off * 3, sl.d_sltpos,
+                                             (size_t)P.desc[i].nins * sl.nslt * 3 * sizeof(float),
+                                             hipMemcpyDeviceToDevice, c->stream));
+                else
+                    src.slot[i] = sl.d_sltpos;
             }
-        hipLaunchKernelGGL(k_prep_sites, dim3((unsigned)((std::max(P.nsite, nslot) + 255) / 256)), dim3(256), 0,
-                           c->stream, P.nsite,
-                           nslot, sd, soln ? (const float *)nullptr : c->d_sltcat.p, c->d_sitepos, c->d_charge.p,
-                           c->d_molbeg.p, soln ? c->d_tag.p : (const int *)nullptr, c->fc, c->K1, c->K2, c->K3,
-                           c->ord, c->d_insposn.p, c->d_insposu.p, c->d_insw.p, c->d_insg.p);
-        HIPCHK(c, hipGetLastError());
-        hipLaunchKernelGGL(k_prep_ins, dim3((unsigned)std::max(1, P.ntot)), dim3(64 * ER_PI_WAVES), 0, c->stream, P.ntot, nslot,
-                           sd, c->fc, c->prm.screen, (int)(c->prm.cltype == 0), c->d_insposn.p, c->d_insref.p,
-                           c->d_selfreal.p, c->d_resself.p);
-        HIPCHK(c, hipGetLastError());
-        const size_t nf = (size_t)P.nsite * (c->H + c->K2 + c->K3);
-        hipLaunchKernelGGL(k_ins_factors, dim3((unsigned)((nf + 255) / 256)), dim3(256), 0, c->stream, P.nsite,
-                           c->ord, c->K1, c->K2, c->K3, c->H, c->d_insposn.p, c->d_insw.p, c->d_insg.p, c->d_tw1.p,
-                           c->d_tw2.p, c->d_tw3.p, c->d_Ftab.p);
-        HIPCHK(c, hipGetLastError());
-        const size_t nC = (size_t)P.ntot * c->ermax;
-        hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)((nC + 255) / 256)), dim3(256), 0, c->stream, nC, c->d_C.p);
-        HIPCHK(c, hipGetLastError());
-        if (c->prm.cltype == 0) {
-            // bare Coulomb (engproc.F90:761-769, 819-826): no reciprocal
-            // part; U starts at zero for the pair sums
-            const size_t n = (size_t)P.ntot * c->nummol;
-            hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, n,
-                               reinterpret_cast<uint32_t *>(c->d_Ucat.p));
-            HIPCHK(c, hipGetLastError());
         }
+        for (const SlotDesc &d : P.desc) maxslt = std::max(maxslt, d.nslt);
+        // four waves per insertion; few insertions of many sites take eight
+        // (a lone 150-site solute among 12 000 waters: 41 us in four, 30 us in eight)
+        const int waves = maxslt > 32 && P.ntot <= 64 ? 8 : 4;
+        const size_t nf = bare ? 0 : (size_t)P.nsite * (c->H + c->K2 + c->K3);
+        const size_t nC = (size_t)P.ntot * c->ermax;
+        // bare Coulomb (engproc.F90:761-769, 819-826): no reciprocal part; U
+        // starts at zero for the pair sums
+        const size_t nU = bare ? (size_t)P.ntot * c->nummol : 0;
+        const size_t fthreads = std::max(nf, std::min<size_t>((nC + nU) / 4 + 1, (size_t)1 << 20));
+        with_order(bare ? 0 : c->ord, [&](auto ord) {
+            constexpr int O = decltype(ord)::value;
+            hipLaunchKernelGGL(k_prep_ins<O>, dim3((unsigned)std::max(1, P.ntot)), dim3(64 * waves), 0, c->stream,
+                               P.ntot, nslot, sd, src, c->d_sitepos, c->d_charge.p, c->d_molbeg.p,
+                               soln ? c->d_tag.p : (const int *)nullptr, c->fc, c->K1, c->K2, c->K3, c->prm.screen,
+                               c->d_insposn.p, c->d_insposu.p, c->d_insw.p, c->d_insg.p, c->d_insref.p,
+                               c->d_selfreal.p, c->d_resself.p);
+            hipLaunchKernelGGL(k_ins_factors<O>, dim3((unsigned)((fthreads + 255) / 256)), dim3(256), 0, c->stream,
+                               P.nsite, c->K1, c->K2, c->K3, c->H, c->d_insposn.p, c->d_insw.p, c->d_insg.p,
+                               c->d_tw1.p, c->d_tw2.p, c->d_tw3.p, c->d_Ftab.p, nC, c->d_C.p, nU,
+                               reinterpret_cast<uint32_t *>(c->d_Ucat.p));
+        });
+        HIPCHK(c, hipGetLastError());
     }
     if (batched) {
         if (c->prm.cltype != 0)
@@ -2842,7 +2878,7 @@ extern "C" int er_set_cell_width(er_ctx *c, float angstrom)
     c->cell_min = angstrom;
     if (c->have_frame && c->prm.boxshp != 0 && c->cell_wmin > 0.0) {
         c->nc = std::max(1, std::min(32, (int)(c->cell_wmin / (c->cell_min > 0.f ? c->cell_min : 3.5f))));
-        c->ncell = morton_keys(c->nc);
+        c->ncell = cell_keys(c->nc);
         c->cell_w = (float)(c->cell_wmin / c->nc);
         c->frame_dirty = true;
     }

@@ -210,24 +210,32 @@ __device__ __forceinline__ float lattice_d2(const FrameConst &fc, const uint4 &a
     return dx * dx + dy * dy + dz * dz;
 }
 
-// B-spline weights w[c] = M_ord(t + c), c = 0..ord-1, by the Cox-de Boor
+// B-spline weights w[c] = M_ORD(t + c), c = 0..ORD-1, by the Cox-de Boor
 // recursion M_k(x) = (x M_{k-1}(x) + (k-x) M_{k-1}(x-1)) / (k-1).  Same
 // values as the explicit sum of spline.F90:46-58 without its cancellation.
-__device__ __forceinline__ void bspline_weights(float t, int ord, float *w)
+// The order is a template argument so that the weights stay in registers (as a
+// run-time order they lived in scratch memory: 90 000 atoms 17 us at order 4,
+// 29 us at order 6).  One fused product per element, as written.
+template <int ORD> __device__ __forceinline__ void bspline_weights(float t, float *w)
 {
+#pragma clang fp contract(off)
     w[0] = t;
     w[1] = 1.0f - t;
-    for (int k = 3; k <= ord; ++k) {
+#pragma unroll
+    for (int k = 3; k <= ORD; ++k) {
         const float inv = 1.0f / (float)(k - 1);
-        w[k - 1] = (1.0f - t) * w[k - 2] * inv;
-        for (int c = k - 2; c >= 1; --c) w[c] = ((t + (float)c) * w[c] + ((float)(k - c) - t) * w[c - 1]) * inv;
-        w[0] = t * w[0] * inv;
+        w[k - 1] = ((1.0f - t) * w[k - 2]) * inv;
+#pragma unroll
+        for (int c = k - 2; c >= 1; --c)
+            w[c] = fmaf(w[c], t + (float)c, ((float)(k - c) - t) * w[c - 1]) * inv;
+        w[0] = (t * w[0]) * inv;
     }
 }
 
 // fractional grid coordinate of one site (recpcal.F90:517-536)
-__device__ __forceinline__ void site_spline(const FrameConst &fc, float x, float y, float z, int K1, int K2,
-                                            int K3, int ord, float *w /*[3*ord]*/, int4 &g)
+template <int ORD>
+__device__ __forceinline__ void site_spline(const FrameConst &fc, float x, float y, float z, int K1, int K2, int K3,
+                                            float *w /*[3*ORD]*/, int4 &g)
 {
     // the fraction and grid coordinate in FP64 from the FP32 position, so
     // that neither carries the rounding of a coordinate as large as the box
@@ -243,7 +251,7 @@ __device__ __forceinline__ void site_spline(const FrameConst &fc, float x, float
         int rci = (int)factor;
         const float t = (float)(factor - (double)rci);
         if (rci >= Ks[k]) rci -= Ks[k];  // a fraction that rounded up to 1
-        bspline_weights(t, ord, w + k * ord);
+        bspline_weights<ORD>(t, w + k * ORD);
         gg[k] = rci;
     }
     g = make_int4(gg[0], gg[1], gg[2], 0);
@@ -253,18 +261,87 @@ __device__ __forceinline__ void site_spline(const FrameConst &fc, float x, float
 // per-frame preparation
 // ---------------------------------------------------------------------------
 
+#ifndef ER_SEG
+#define ER_SEG 8  // atoms per molecule segment of the pair search's pruning
+#endif
+
+// centroid of the sites P(a0) .. P(a1 - 1) (minimum-image offsets from the
+// first, averaged) and their largest minimum-image distance from it: a sphere
+// that holds every site, for the pair search's pruning (any centre is valid
+// by the triangle inequality on minimum images; the centroid reaches least
+// far for extended molecules).  G lanes (a power of two, neighbours in the
+// wave) share the sites, lane l of them taking every G-th.
+template <class POS>
+__device__ __forceinline__ float4 site_sphere(const FrameConst &fc, POS P, int a0, int a1, int l, int G)
+{
+    const float4 r = P(a0);
+    float ox = 0.0f, oy = 0.0f, oz = 0.0f;
+    for (int a = a0 + l; a < a1; a += G) {
+        const float4 p = P(a);
+        float dx = p.x - r.x, dy = p.y - r.y, dz = p.z - r.z;
+        min_image(fc, dx, dy, dz);
+        ox += dx;
+        oy += dy;
+        oz += dz;
+    }
+    for (int off = G >> 1; off > 0; off >>= 1) {
+        ox += __shfl_xor(ox, off, 64);
+        oy += __shfl_xor(oy, off, 64);
+        oz += __shfl_xor(oz, off, 64);
+    }
+    const float inv = 1.0f / (float)(a1 - a0);
+    const float cx = r.x + ox * inv, cy = r.y + oy * inv, cz = r.z + oz * inv;
+    float R = 0.0f;
+    for (int a = a0 + l; a < a1; a += G) {
+        const float4 p = P(a);
+        float dx = p.x - cx, dy = p.y - cy, dz = p.z - cz;
+        min_image(fc, dx, dy, dz);
+        R = fmaxf(R, sqrtf(dx * dx + dy * dy + dz * dz));
+    }
+    for (int off = G >> 1; off > 0; off >>= 1) R = fmaxf(R, __shfl_xor(R, off, 64));
+    return make_float4(cx, cy, cz, R);
+}
+
 // realcal_prepare (realcal.F90:30-48) + recpcal_prepare_solvent
-// (recpcal.F90:340-357) for every physical atom
-// The frame's sort counters (cell counts, brick counts and the largest
-// molecule reach) are cleared here too, before the kernels that add to them.
-__global__ void k_prep_atoms(int natom, const float *__restrict__ pos, const float *__restrict__ charge,
-                             FrameConst fc, int K1, int K2, int K3, int ord, float4 *__restrict__ posn,
-                             uint4 *__restrict__ posu, float *__restrict__ splw, int4 *__restrict__ splg,
-                             unsigned int *__restrict__ ccnt, int ncell, unsigned int *__restrict__ bcnt, int nbrick,
-                             float *__restrict__ rmolmax)
+// (recpcal.F90:340-357) for every physical atom (blocks [0, nab)), and the
+// bounding sphere of every molecule and of each of its segments of ER_SEG
+// consecutive atoms (stored at the segment's first atom in segref; the blocks
+// after them, G = 2^gsh lanes per molecule).  The molecule blocks read the
+// positions as the atoms' blocks do, so that one launch serves both.  ORD 0:
+// no reciprocal part, no splines.  The frame's sort counters (cell and
+// brick counts, the largest molecule reach) are cleared here, before the kernel
+// that adds to them.
+// Latency-bound: a dependent load and an FP64 chain per site.  A 150-atom
+// molecule took one thread 89 us; with 16 lanes it hides under the atoms.
+template <int ORD>
+__global__ void __launch_bounds__(256) k_prep_frame(int natom, int nab, const float *__restrict__ pos,
+                                                    const float *__restrict__ charge, FrameConst fc, int K1, int K2,
+                                                    int K3, float4 *__restrict__ posn, uint4 *__restrict__ posu,
+                                                    float *__restrict__ splw, int4 *__restrict__ splg,
+                                                    unsigned int *__restrict__ ccnt, int ncell,
+                                                    unsigned int *__restrict__ bcnt, int nbrick,
+                                                    float *__restrict__ rmolmax, int nmol, int gsh,
+                                                    const int *__restrict__ molbeg, float4 *__restrict__ molref,
+                                                    float4 *__restrict__ segref)
 {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    const int T = gridDim.x * blockDim.x;
+    if ((int)blockIdx.x >= nab) {
+        const int t = a - nab * (int)blockDim.x, G = 1 << gsh;
+        const int j = t >> gsh, l = t & (G - 1);
+        if (j >= nmol) return;  // whole groups: nmol G lanes
+        auto P = [&](int i) {
+            float x = pos[3 * (size_t)i], y = pos[3 * (size_t)i + 1], z = pos[3 * (size_t)i + 2];
+            rotate_site(fc, x, y, z);
+            return make_float4(x, y, z, 0.0f);
+        };
+        const int a0 = molbeg[j], a1 = molbeg[j + 1];
+        const float4 ms = site_sphere(fc, P, a0, a1, l, G);
+        if (l == 0) molref[j] = ms;
+        for (int s0 = a0 + l * ER_SEG; s0 < a1; s0 += G * ER_SEG)
+            segref[s0] = site_sphere(fc, P, s0, min(s0 + ER_SEG, a1), 0, 1);
+        return;
+    }
+    const int T = nab * blockDim.x;
     for (int i = a; i < ncell; i += T) ccnt[i] = 0u;
     for (int i = a; i < nbrick; i += T) bcnt[i] = 0u;
     if (a == 0) *rmolmax = 0.0f;
@@ -274,127 +351,57 @@ __global__ void k_prep_atoms(int natom, const float *__restrict__ pos, const flo
     rotate_site(fc, wx, wy, wz);
     posn[a] = make_float4(wx, wy, wz, charge[a]);
     posu[a] = lattice_site(fc, x, y, z, charge[a]);
-    float w[3 * ER_MAXORD];
-    int4 g;
-    site_spline(fc, x, y, z, K1, K2, K3, ord, w, g);
-    for (int k = 0; k < 3 * ord; ++k) splw[(size_t)a * 3 * ord + k] = w[k];
-    splg[a] = g;
+    if constexpr (ORD > 0) {
+        float w[3 * ORD];
+        int4 g;
+        site_spline<ORD>(fc, x, y, z, K1, K2, K3, w, g);
+#pragma unroll
+        for (int k = 0; k < 3 * ORD; ++k) splw[(size_t)a * 3 * ORD + k] = w[k];
+        splg[a] = g;
+    }
 }
 
-// centre and reach radius of each molecule (for cutoff pruning)
-#ifndef ER_SEG
-#define ER_SEG 8  // atoms per molecule segment of the pair search's pruning
-#endif
+// The solutes' insertion coordinates of a run, by slot; beyond ER_INS_PTRS
+// slots they are copied end to end first (cat).
+#define ER_INS_PTRS 16
+struct InsSource {
+    const float *slot[ER_INS_PTRS];
+    const float *cat;
+};
 
-// centroid of the atoms [a0, a1) (minimum-image offsets from atom a0,
-// averaged) and their largest minimum-image distance from it: a sphere that
-// holds every atom, for the pair search's pruning (any centre is valid by
-// the triangle inequality on minimum images; the centroid reaches least far
-// for extended molecules)
-__device__ __forceinline__ float4 atom_sphere(const FrameConst &fc, const float4 *__restrict__ posn, int a0, int a1)
+// One workgroup per insertion (refs) or solute molecule (soln): its sites'
+// position, lattice coordinates and spline, then the pair search's centre and
+// reach radius, the real-space self energy realcal_self[_refs]
+// (realcal.F90:669-771) and the residual self term.  Block 0 counts the run for
+// every solute (the run number of the halt keys, read by the histograms later
+// in the run).
+// Bound by the FP64 erf chain of the self energy: its pairs go round
+// ER_PI_PART partial sums, dealt to the threads and added in one order whatever
+// the wave count, so a lone 150-site solute can take eight waves (30 us;
+// 64 us for the sites and the self energy in four waves).
+#define ER_PI_ROWS 512   // sites held in LDS
+#define ER_PI_PART 1024  // partial sums of the self energy
+template <int ORD>
+__global__ void __launch_bounds__(512) k_prep_ins(int ntot, int nslot, const SlotDesc *__restrict__ sd,
+                                                   InsSource src, const float *__restrict__ frame_pos,
+                                                   const float *__restrict__ charge, const int *__restrict__ molbeg,
+                                                   const int *__restrict__ tag, FrameConst fc, int K1, int K2, int K3,
+                                                   float screen, float4 *insposn, uint4 *__restrict__ insposu,
+                                                   float *__restrict__ insw, int4 *__restrict__ insg,
+                                                   float4 *__restrict__ insref, float *__restrict__ selfreal,
+                                                   float *__restrict__ resself)
 {
-    const float4 r = posn[a0];
-    float ox = 0.0f, oy = 0.0f, oz = 0.0f;
-    for (int a = a0 + 1; a < a1; ++a) {
-        const float4 p = posn[a];
-        float dx = p.x - r.x, dy = p.y - r.y, dz = p.z - r.z;
-        min_image(fc, dx, dy, dz);
-        ox += dx;
-        oy += dy;
-        oz += dz;
-    }
-    const float inv = 1.0f / (float)(a1 - a0);
-    const float cx = r.x + ox * inv, cy = r.y + oy * inv, cz = r.z + oz * inv;
-    float R = 0.0f;
-    for (int a = a0; a < a1; ++a) {
-        const float4 p = posn[a];
-        float dx = p.x - cx, dy = p.y - cy, dz = p.z - cz;
-        min_image(fc, dx, dy, dz);
-        R = fmaxf(R, sqrtf(dx * dx + dy * dy + dz * dz));
-    }
-    return make_float4(cx, cy, cz, R);
-}
-
-// Per molecule: its bounding sphere (atom_sphere), and for every segment of
-// ER_SEG consecutive atoms (molecule-relative) the segment's, stored at the
-// segment's first atom in segref
-__global__ void k_prep_mols(int nmol, const int *__restrict__ molbeg, const float4 *__restrict__ posn,
-                            FrameConst fc, float4 *__restrict__ molref, float *__restrict__ rmolmax,
-                            float4 *__restrict__ segref)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= nmol) return;
-    const int a0 = molbeg[j], a1 = molbeg[j + 1];
-    const float4 ms = atom_sphere(fc, posn, a0, a1);
-    const float R = ms.w;
-    molref[j] = ms;
-    for (int s0 = a0; s0 < a1; s0 += ER_SEG) {
-        segref[s0] = atom_sphere(fc, posn, s0, min(s0 + ER_SEG, a1));
-    }
-    // frame maximum (non-negative floats order like their bit patterns)
-    atomicMax(reinterpret_cast<unsigned int *>(rmolmax), __float_as_uint(R));
-}
-
-// Insertion (refs) or solute molecule (soln) sites: position, lattice
-// coordinates and spline; k_prep_ins then adds the search sphere and the real-space self term
-// realcal_self[_refs] (realcal.F90:669-771).  For soln the sites come from
-// the frame.
-__global__ void k_prep_sites(int nsite, int nslot, const SlotDesc *__restrict__ sd, const float *__restrict__ sltpos,
-                             const float *__restrict__ frame_pos, const float *__restrict__ charge,
-                             const int *__restrict__ molbeg, const int *__restrict__ tag, FrameConst fc, int K1,
-                             int K2, int K3, int ord, float4 *__restrict__ insposn, uint4 *__restrict__ insposu,
-                             float *__restrict__ insw, int4 *__restrict__ insg)
-{
-    // one thread per site of the run (every solute's insertions end to end):
-    // spline weights, grid base, position and lattice coordinates.  The
-    // first nslot threads also count the run for their solute (the run
-    // number of the halt keys, read by the histograms later in the run).
-    const int is = blockIdx.x * blockDim.x + threadIdx.x;
-    if (is < nslot) *sd[is].seq += 1u;
-    if (is >= nsite) return;
-    const int k = slot_find(nslot, is, [&](int m) { return sd[m].site_off; });
-    const int nslt = sd[k].nslt;
-    const int local = is - sd[k].site_off;
-    const int n = local / nslt, s = local % nslt;
-    float x, y, z, q;
-    if (tag) {  // soln: the solute molecules' sites from the frame
-        const size_t a = (size_t)molbeg[tag[n]] + s;
-        x = frame_pos[3 * a]; y = frame_pos[3 * a + 1]; z = frame_pos[3 * a + 2];
-        q = charge[a];
-    } else {  // refs: the run's insertion coordinates, solutes end to end
-        const size_t o = (size_t)is * 3;
-        x = sltpos[o]; y = sltpos[o + 1]; z = sltpos[o + 2];
-        q = sd[k].sltq[s];
-    }
-    float w[3 * ER_MAXORD];
-    int4 g;
-    site_spline(fc, x, y, z, K1, K2, K3, ord, w, g);
-    for (int c = 0; c < 3 * ord; ++c) insw[(size_t)is * 3 * ord + c] = w[c];
-    insg[is] = g;
-    insposu[is] = lattice_site(fc, x, y, z, q);
-    rotate_site(fc, x, y, z);
-    insposn[is] = make_float4(x, y, z, q);
-}
-
-// One workgroup of four waves per insertion (after k_prep_sites): search
-// centre and reach radius (every wave computes them; wave 0 writes), the
-// real-space self energy with the site pairs shared by the four waves, and
-// the residual self term.
-#define ER_PI_WAVES 4
-__global__ void __launch_bounds__(64 * ER_PI_WAVES) k_prep_ins(int ntot, int nslot, const SlotDesc *__restrict__ sd,
-                                                               FrameConst fc, float screen, int bare,
-                                                               const float4 *__restrict__ insposn,
-                                                               float4 *__restrict__ insref,
-                                                               float *__restrict__ selfreal,
-                                                               float *__restrict__ resself)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ float4 sP[ER_PI_ROWS];
+    __shared__ double part[ER_PI_PART];
+    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wave = tid >> 6;
     const int n = blockIdx.x;
+    if (n == 0)
+        for (int k = tid; k < nslot; k += NT) *sd[k].seq += 1u;
     if (n >= ntot) return;
     const int k = ER_SLOT_OF_INS(sd, nslot, n);
     const int local = n - sd[k].ins_off;
     if (local >= sd[k].nins) {  // padding of the solute's insertion range
-        if (threadIdx.x == 0) {
+        if (tid == 0) {
             insref[n] = make_float4(0.f, 0.f, 0.f, 0.f);
             selfreal[n] = 0.0f;
             resself[n] = 0.0f;
@@ -402,40 +409,40 @@ __global__ void __launch_bounds__(64 * ER_PI_WAVES) k_prep_ins(int ntot, int nsl
         return;
     }
     const int nslt = sd[k].nslt;
-    const float4 *P = insposn + sd[k].site_off + (size_t)local * nslt;
-    // The pair search's centre: the sites' centroid (their minimum-image
-    // offsets from site 0, averaged), with reach R = the largest minimum-image
-    // distance of a site from it.  Any centre bounds the search by the
-    // triangle inequality on minimum images; the centroid of an extended
-    // solute reaches far less than its first site (28 -> ~16 A for a
-    // 150-site chain), and the search volume goes with the cube of cutoff +
-    // reach.
-    const float4 c0 = P[0];
-    float ox = 0.0f, oy = 0.0f, oz = 0.0f;
-    for (int s = 1 + lane; s < nslt; s += 64) {
-        float dx = P[s].x - c0.x, dy = P[s].y - c0.y, dz = P[s].z - c0.z;
-        min_image(fc, dx, dy, dz);
-        ox += dx;
-        oy += dy;
-        oz += dz;
+    const size_t row = (size_t)sd[k].site_off + (size_t)local * nslt;
+    const float *sltq = sd[k].sltq;
+    const size_t atom0 = tag ? (size_t)molbeg[tag[n]] : 0;
+    // soln: the solute molecule's sites from the frame; refs: the coordinates given
+    const float *from = tag ? frame_pos + 3 * atom0
+                            : (src.cat ? src.cat + 3 * row : src.slot[k] + (size_t)local * nslt * 3);
+    for (int s = tid; s < nslt; s += NT) {
+        float x = from[3 * (size_t)s], y = from[3 * (size_t)s + 1], z = from[3 * (size_t)s + 2];
+        const float q = tag ? charge[atom0 + s] : sltq[s];
+        insposu[row + s] = lattice_site(fc, x, y, z, q);
+        if constexpr (ORD > 0) {
+            float w[3 * ORD];
+            int4 g;
+            site_spline<ORD>(fc, x, y, z, K1, K2, K3, w, g);
+#pragma unroll
+            for (int c = 0; c < 3 * ORD; ++c) insw[(row + s) * 3 * ORD + c] = w[c];
+            insg[row + s] = g;
+        }
+        rotate_site(fc, x, y, z);
+        const float4 p = make_float4(x, y, z, q);
+        insposn[row + s] = p;
+        if (s < ER_PI_ROWS) sP[s] = p;
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        ox += __shfl_xor(ox, off, 64);
-        oy += __shfl_xor(oy, off, 64);
-        oz += __shfl_xor(oz, off, 64);
-    }
-    const float inv = 1.0f / (float)nslt;
-    const float cx = c0.x + ox * inv, cy = c0.y + oy * inv, cz = c0.z + oz * inv;
-    float R = 0.0f;
-    for (int s = lane; s < nslt; s += 64) {
-        float dx = P[s].x - cx, dy = P[s].y - cy, dz = P[s].z - cz;
-        min_image(fc, dx, dy, dz);
-        R = fmaxf(R, sqrtf(dx * dx + dy * dy + dz * dz));
-    }
-    for (int off = 32; off > 0; off >>= 1) R = fmaxf(R, __shfl_xor(R, off, 64));
-    if (bare) {  // cltype 0: realcal_self and residual_self_ene return at once
-        if (threadIdx.x == 0) {
-            insref[n] = make_float4(cx, cy, cz, R);
+    __syncthreads();
+    const bool in_lds = nslt <= ER_PI_ROWS;
+    auto P = [&](int s) { return in_lds ? sP[s] : insposn[row + s]; };
+    // The pair search's centre: the sites' centroid, reach R (every wave
+    // computes them).  The centroid of an extended solute reaches far less than
+    // its first site (28 -> ~16 A for a 150-site chain), and the search volume
+    // goes with the cube of cutoff + reach.
+    const float4 sph = site_sphere(fc, P, 0, nslt, lane, 64);
+    if (ORD == 0) {  // cltype 0: realcal_self and residual_self_ene return at once
+        if (tid == 0) {
+            insref[n] = sph;
             selfreal[n] = 0.0f;
             resself[n] = 0.0f;
         }
@@ -444,38 +451,41 @@ __global__ void __launch_bounds__(64 * ER_PI_WAVES) k_prep_ins(int ntot, int nsl
     // realcal_self_refs: -sum q^2 alpha/sqrt(pi) - sum_{i<j} q_i q_j erf(alpha r)/r,
     // in FP64 from the FP32 positions and charges: a 150-site solute has
     // 11 175 terms of up to tens of kcal/mol that largely cancel, and this
-    // self energy enters the insertion's weight; computed once per
-    // insertion, FP64 costs little here.  Wave w takes the rows s = w mod 4
-    // and its lane l the pairs (s, t) with t - s - 1 = l mod 64, then a
-    // fixed-order tree in each wave and the four waves added in order.
-    double e = 0.0;
+    // self energy enters the insertion's weight
     const double rsqpi = 0.564189583547756286948079451560772586;  // 1/sqrt(pi)
     const double scr = screen;
-    if (wave == 0)
-        for (int s = lane; s < nslt; s += 64) e += -(double)P[s].w * (double)P[s].w * scr * rsqpi;
-    for (int s = wave; s < nslt; s += ER_PI_WAVES) {
-        const float4 a = P[s];
-        for (int t = s + 1 + lane; t < nslt; t += 64) {
-            const float4 b = P[t];
+    // the pairs (s < t) as a rectangle: row r holds the pairs of site r and
+    // then those of site n - 1 - r (n - 2 - r for odd n)
+    const int L = (nslt & 1) ? nslt : nslt - 1, np = (nslt >> 1) * L;
+    for (int v = tid; v < ER_PI_PART; v += NT) {
+        double ev = 0.0;
+        for (int i = v; i < np; i += ER_PI_PART) {
+            const int r = i / L, c = i - r * L, len = nslt - 1 - r;
+            const int s1 = c < len ? r : ((nslt & 1) ? nslt - 2 - r : nslt - 1 - r);
+            const int t1 = c < len ? r + 1 + c : s1 + 1 + (c - len);
+            const float4 a = P(s1), b = P(t1);
             double dx = (double)a.x - (double)b.x, dy = (double)a.y - (double)b.y, dz = (double)a.z - (double)b.z;
             min_image_d(fc, dx, dy, dz);
-            const double r = sqrt(dx * dx + dy * dy + dz * dz);
-            e += -(double)a.w * (double)b.w * erf(scr * r) / r;
+            const double rr = sqrt(dx * dx + dy * dy + dz * dz);
+            ev += -(double)a.w * (double)b.w * erf(scr * rr) / rr;
         }
+        part[v] = ev;
     }
-    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
-    __shared__ double wsum[ER_PI_WAVES];
-    if (lane == 0) wsum[wave] = e;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        e = wsum[0];
-        for (int w = 1; w < ER_PI_WAVES; ++w) e += wsum[w];
-        insref[n] = make_float4(cx, cy, cz, R);
+    double e = 0.0;
+    if (wave == 0) {
+        for (int s = lane; s < nslt; s += 64) e += -(double)P(s).w * (double)P(s).w * scr * rsqpi;
+        for (int v = lane; v < min(np, ER_PI_PART); v += 64) e += part[v];
+    }
+    if (wave != 0) return;
+    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
+    if (lane == 0) {
+        insref[n] = sph;
         selfreal[n] = (float)e;
         // residual_self_ene (engproc.F90:967-977): -(pi Q^2 / alpha^2 / V) / 2 with
         // Q = mol_charge, a plain sum of the site charges (setconf.F90:838-840)
         float Q = 0.0f;
-        for (int s = 0; s < nslt; ++s) Q += P[s].w;
+        for (int s = 0; s < nslt; ++s) Q += P(s).w;
         float epcl = ER_PI_F * Q * Q / screen / screen / fc.volume;
         epcl = epcl / 2.0f;
         resself[n] = 0.0f - epcl;
@@ -608,37 +618,51 @@ __host__ __device__ constexpr int tws_off(int r) { return r * (r - 1) / 2 - 6; }
 // per run instead of once per (insertion, m1) plane:
 //   F_axis(m) = sum_c w_c exp(-2 pi i m (g - c) / K)   (axis 1 scaled by q)
 // Ftab: [insertion][site][H + K2 + K3]: m1 = 0..H-1, then m2, then m3.
-__global__ void k_ins_factors(int nrows, int ord, int K1, int K2, int K3, int H,
-                              const float4 *__restrict__ insposn, const float *__restrict__ insw,
-                              const int4 *__restrict__ insg, const float2 *__restrict__ tw1,
-                              const float2 *__restrict__ tw2, const float2 *__restrict__ tw3,
-                              float2 *__restrict__ Ftab)
+// The launch also clears the run's counts (nC words at C) and, without a
+// reciprocal part (nrows 0), the energies the pair search adds to (nU words).
+template <int ORD>
+__global__ void __launch_bounds__(256) k_ins_factors(int nrows, int K1, int K2, int K3, int H,
+                                                     const float4 *__restrict__ insposn,
+                                                     const float *__restrict__ insw, const int4 *__restrict__ insg,
+                                                     const float2 *__restrict__ tw1, const float2 *__restrict__ tw2,
+                                                     const float2 *__restrict__ tw3, float2 *__restrict__ Ftab,
+                                                     size_t nC, uint32_t *__restrict__ C, size_t nU,
+                                                     uint32_t *__restrict__ U)
 {
-    const int per = H + K2 + K3;
-    const size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= (size_t)nrows * per) return;
-    const int r = (int)(f % per);
-    const size_t site = f / per;
-    const int4 g = insg[site];
-    int axis, m, K, gd;
-    const float2 *tw;
-    if (r < H) { axis = 0; m = r; K = K1; gd = g.x; tw = tw1; }
-    else if (r < H + K2) { axis = 1; m = r - H; K = K2; gd = g.y; tw = tw2; }
-    else { axis = 2; m = r - H - K2; K = K3; gd = g.z; tw = tw3; }
-    const float *w = insw + site * 3 * ord + axis * ord;
-    float2 a = make_float2(0.f, 0.f);
-    // e = m (g - c) mod K: one reduction for c = 0 (m, pmod(.) < K <= 512, so
-    // the product fits 32 bits), then e - m mod K for each next c
-    int e = (int)(((unsigned int)m * (unsigned int)pmod(gd, K)) % (unsigned int)K);
-    for (int c = 0; c < ord; ++c) {
-        const float2 t = tw[e];  // exp(+2 pi i e/K); the forward sum uses the conjugate
-        a.x += w[c] * t.x;
-        a.y -= w[c] * t.y;
-        e -= m;
-        e += (e < 0) ? K : 0;
+    const size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x, T = (size_t)gridDim.x * blockDim.x;
+    auto clear = [&](size_t n, uint32_t *p) {
+        for (size_t i = f; i < n / 4; i += T) reinterpret_cast<uint4 *>(p)[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (f < n % 4) p[n / 4 * 4 + f] = 0u;
+    };
+    clear(nC, C);
+    if (nU) clear(nU, U);
+    if constexpr (ORD > 0) {
+        const int per = H + K2 + K3;
+        if (f >= (size_t)nrows * per) return;
+        const int r = (int)(f % per);
+        const size_t site = f / per;
+        const int4 g = insg[site];
+        int axis, m, K, gd;
+        const float2 *tw;
+        if (r < H) { axis = 0; m = r; K = K1; gd = g.x; tw = tw1; }
+        else if (r < H + K2) { axis = 1; m = r - H; K = K2; gd = g.y; tw = tw2; }
+        else { axis = 2; m = r - H - K2; K = K3; gd = g.z; tw = tw3; }
+        const float *w = insw + site * 3 * ORD + axis * ORD;
+        float2 a = make_float2(0.f, 0.f);
+        // e = m (g - c) mod K: one reduction for c = 0 (m, pmod(.) < K <= 512, so
+        // the product fits 32 bits), then e - m mod K for each next c
+        int e = (int)(((unsigned int)m * (unsigned int)pmod(gd, K)) % (unsigned int)K);
+#pragma unroll
+        for (int c = 0; c < ORD; ++c) {
+            const float2 t = tw[e];  // exp(+2 pi i e/K); the forward sum uses the conjugate
+            a.x += w[c] * t.x;
+            a.y -= w[c] * t.y;
+            e -= m;
+            e += (e < 0) ? K : 0;
+        }
+        if (axis == 0) a = erfft::cscale(a, insposn[site].w);
+        Ftab[f] = a;
     }
-    if (axis == 0) a = erfft::cscale(a, insposn[site].w);
-    Ftab[f] = a;
 }
 
 // One term engfac(m) |rho^(m)|^2 of the half-plane self energy
@@ -1377,18 +1401,21 @@ __global__ void __launch_bounds__(ER_GEN_NT) k_pme_axis1_gen(int nchunk, int NI,
 // molecules in this order (neighbouring stencils hit the same L2 lines) and
 // the pair search uses the cells as a cell list.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ unsigned int morton_spread(unsigned int v)  // 10 bits -> every third bit
+// key of cell (cx, cy, cz) of nc^3: blocks of 4 x 4 x 4 cells in rows, Morton
+// order inside a block, ceil(nc / 4)^3 64 keys in all (a Morton code over
+// the whole grid takes 32768 keys from nc = 17 on: the scan of 17^3 cells took
+// 10 us)
+__host__ __device__ __forceinline__ int cell_keys(int nc)
 {
-    v &= 0x3ffu;
-    v = (v | (v << 16)) & 0x030000ffu;
-    v = (v | (v << 8)) & 0x0300f00fu;
-    v = (v | (v << 4)) & 0x030c30c3u;
-    v = (v | (v << 2)) & 0x09249249u;
-    return v;
+    const int nb = (nc + 3) / 4;
+    return nb * nb * nb * 64;
 }
-__device__ __forceinline__ unsigned int cell_key(int cx, int cy, int cz)
+__device__ __forceinline__ unsigned int cell_key(int cx, int cy, int cz, int nc)
 {
-    return morton_spread(cx) | (morton_spread(cy) << 1) | (morton_spread(cz) << 2);
+    const int nb = (nc + 3) >> 2;
+    const unsigned int blk = ((cz >> 2) * nb + (cy >> 2)) * nb + (cx >> 2);
+    auto pair = [](int v) { return (unsigned int)((v & 1) | (v & 2) << 2); };  // bits 0 and 3
+    return blk << 6 | pair(cx) | pair(cy) << 1 | pair(cz) << 2;
 }
 // fractional position of a wrapped site -> cell coordinate in [0, nc)
 __device__ __forceinline__ void site_cell(const FrameConst &fc, float x, float y, float z, int nc, int &cx, int &cy,
@@ -1405,62 +1432,114 @@ __device__ __forceinline__ void site_cell(const FrameConst &fc, float x, float y
     cz = min(nc - 1, (int)(u[2] * nc));
 }
 
-// the two counting passes of the frame's sorts in one launch: threads
-// [0, nmol) count the molecules per cell (the molecule centre's cell), the
-// next natom threads the atoms per PME brick (the brick of the spline base)
-__global__ void k_sort_count(int nmol, const float4 *__restrict__ molref, FrameConst fc, int nc,
-                             unsigned int *__restrict__ ccnt, unsigned int *__restrict__ keyrank, int natom,
-                             const int4 *__restrict__ splg, int K1, int K2, int K3, int nbx, int nby, int bzs,
-                             unsigned int *__restrict__ bcnt, unsigned int *__restrict__ akeyrank)
+// a molecule's cell and an atom's PME brick
+struct SortGrid {
+    int nc, K1, K2, K3, nbx, nby, bzs, nbrick;
+};
+__device__ __forceinline__ unsigned int mol_cell(const FrameConst &fc, const SortGrid &sg, const float4 &m)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < nmol) {
-        const float4 m = molref[t];
-        int cx, cy, cz;
-        site_cell(fc, m.x, m.y, m.z, nc, cx, cy, cz);
-        const unsigned int key = cell_key(cx, cy, cz);
-        const unsigned int rank = atomicAdd(&ccnt[key], 1u);
-        keyrank[2 * t] = key;
-        keyrank[2 * t + 1] = rank;
-        return;
-    }
-    const int a = t - nmol;
-    if (a >= natom) return;
-    const int4 g = splg[a];
-    const unsigned int key = (unsigned int)((pmod(g.z, K3) / bzs * nby + pmod(g.y, K2) / ER_BRICK) * nbx +
-                                            pmod(g.x, K1) / ER_BRICK);
-    akeyrank[2 * a] = key;
-    akeyrank[2 * a + 1] = atomicAdd(&bcnt[key], 1u);
+    int cx, cy, cz;
+    site_cell(fc, m.x, m.y, m.z, sg.nc, cx, cy, cz);
+    return cell_key(cx, cy, cz, sg.nc);
+}
+__device__ __forceinline__ unsigned int atom_brick(const SortGrid &sg, const int4 &g)
+{
+    return (unsigned int)((pmod(g.z, sg.K3) / sg.bzs * sg.nby + pmod(g.y, sg.K2) / ER_BRICK) * sg.nbx +
+                          pmod(g.x, sg.K1) / ER_BRICK);
 }
 
-// exclusive scan of n counts by one 1024-thread block -> start[n + 1]:
-// each thread scans ER_SCAN_CH consecutive counts in registers, the thread
-// totals go through one wave scan and one LDS exchange, so a 32768-count
-// scan takes a single pass of two barriers
-#define ER_SCAN_CH 32
-__device__ __forceinline__ void block_scan(int ncell, const unsigned int *__restrict__ cnt,
+// The two counting passes of the frame's sorts in one launch: blocks [0, nmb)
+// count the molecules per cell and find the largest molecule reach, the others
+// the atoms per PME brick, ER_SORT_APT per thread.  A device atomic costs a
+// trip beyond the XCD's L2 and atoms far outnumber bricks, so a block counts
+// its atoms in LDS first and adds one total per brick (90 000 atoms on 972
+// bricks: 30 us with an atomic per atom, 11 us).  More bricks than
+// ER_SORT_LDS: an atomic per atom.
+#define ER_SORT_APT 4
+#define ER_SORT_LDS 8192
+__global__ void __launch_bounds__(1024) k_sort_count(int nmol, int nmb, const float4 *__restrict__ molref,
+                                                     FrameConst fc, SortGrid sg, unsigned int *__restrict__ ccnt,
+                                                     unsigned int *__restrict__ keyrank, float *__restrict__ rmolmax,
+                                                     int natom, const int4 *__restrict__ splg,
+                                                     unsigned int *__restrict__ bcnt,
+                                                     unsigned int *__restrict__ akeyrank)
+{
+    extern __shared__ __align__(16) unsigned int lcnt[];
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x < nmb) {
+        const int t = blockIdx.x * 1024 + tid;
+        float R = 0.0f;
+        if (t < nmol) {
+            const float4 m = molref[t];
+            const unsigned int key = mol_cell(fc, sg, m);
+            keyrank[2 * t] = key;
+            keyrank[2 * t + 1] = atomicAdd(&ccnt[key], 1u);
+            R = m.w;
+        }
+        // frame maximum (non-negative floats order like their bit patterns)
+        for (int off = 32; off > 0; off >>= 1) R = fmaxf(R, __shfl_xor(R, off, 64));
+        if ((tid & 63) == 0) atomicMax(reinterpret_cast<unsigned int *>(rmolmax), __float_as_uint(R));
+        return;
+    }
+    const bool lds = sg.nbrick <= ER_SORT_LDS;
+    unsigned int *cnt = lds ? lcnt : bcnt;
+    if (lds) {
+        for (int b = tid; b < sg.nbrick; b += 1024) lcnt[b] = 0u;
+        __syncthreads();
+    }
+    const int a0 = ((int)blockIdx.x - nmb) * 1024 * ER_SORT_APT + tid;
+    unsigned int key[ER_SORT_APT], rank[ER_SORT_APT];
+#pragma unroll
+    for (int k = 0; k < ER_SORT_APT; ++k) {
+        const int a = a0 + k * 1024;
+        key[k] = a < natom ? atom_brick(sg, splg[a]) : 0u;
+        rank[k] = a < natom ? atomicAdd(&cnt[key[k]], 1u) : 0u;
+    }
+    if (lds) {
+        __syncthreads();
+        for (int b = tid; b < sg.nbrick; b += 1024) {
+            const unsigned int c = lcnt[b];
+            if (c) lcnt[b] = atomicAdd(&bcnt[b], c);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < ER_SORT_APT; ++k) {
+        const int a = a0 + k * 1024;
+        if (a >= natom) continue;
+        akeyrank[2 * a] = key[k];
+        akeyrank[2 * a + 1] = rank[k] + (lds ? lcnt[key[k]] : 0u);
+    }
+}
+
+// exclusive scan of n counts by one block of NT threads -> start[n + 1]:
+// each thread scans CH consecutive counts in registers, the thread
+// totals go through one wave scan and one LDS exchange, so a pass of NT CH
+// counts takes two barriers
+template <int CH, int NT>
+__device__ __forceinline__ void block_scan(int ncell, const unsigned int *cnt,
                                            unsigned int *__restrict__ start, unsigned int *wsum)
 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     unsigned int carry = 0;
-    for (int base = 0; base < ncell; base += 1024 * ER_SCAN_CH) {
-        const int b0 = base + tid * ER_SCAN_CH;
-        const bool whole = b0 + ER_SCAN_CH <= ncell;  // the thread's counts lie inside the array
-        unsigned int v[ER_SCAN_CH];
+    for (int base = 0; base < ncell; base += NT * CH) {
+        const int b0 = base + tid * CH;
+        const bool whole = b0 + CH <= ncell;  // the thread's counts lie inside the array
+        unsigned int v[CH];
         unsigned int sum = 0;
-        if (whole) {  // 16-byte loads (b0 is a multiple of 32, the array 256-byte aligned)
+        if (whole) {  // 16-byte loads (b0 is a multiple of CH, the array 256-byte aligned)
             const uint4 *c4 = reinterpret_cast<const uint4 *>(cnt + b0);
 #pragma unroll
-            for (int q = 0; q < ER_SCAN_CH / 4; ++q) {
+            for (int q = 0; q < CH / 4; ++q) {
                 const uint4 t = c4[q];
                 v[4 * q] = t.x; v[4 * q + 1] = t.y; v[4 * q + 2] = t.z; v[4 * q + 3] = t.w;
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < ER_SCAN_CH; ++k) v[k] = (b0 + k < ncell) ? cnt[b0 + k] : 0u;
+            for (int k = 0; k < CH; ++k) v[k] = (b0 + k < ncell) ? cnt[b0 + k] : 0u;
         }
 #pragma unroll
-        for (int k = 0; k < ER_SCAN_CH; ++k) sum += v[k];
+        for (int k = 0; k < CH; ++k) sum += v[k];
         unsigned int x = sum;  // inclusive scan of the thread totals over the wave
         for (int off = 1; off < 64; off <<= 1) {
             const unsigned int y = __shfl_up(x, off, 64);
@@ -1469,7 +1548,7 @@ __device__ __forceinline__ void block_scan(int ncell, const unsigned int *__rest
         if (lane == 63) wsum[wave] = x;
         __syncthreads();
         unsigned int before = 0, total = 0;
-        for (int w = 0; w < 16; ++w) {
+        for (int w = 0; w < NT / 64; ++w) {
             const unsigned int t = wsum[w];
             before += (w < wave) ? t : 0u;
             total += t;
@@ -1478,7 +1557,7 @@ __device__ __forceinline__ void block_scan(int ncell, const unsigned int *__rest
         if (whole) {  // start[] holds ncell + 1 entries: the 16-byte stores stay inside
             uint4 *s4 = reinterpret_cast<uint4 *>(start + b0);
 #pragma unroll
-            for (int q = 0; q < ER_SCAN_CH / 4; ++q) {
+            for (int q = 0; q < CH / 4; ++q) {
                 uint4 t;
                 t.x = run; run += v[4 * q];
                 t.y = run; run += v[4 * q + 1];
@@ -1488,7 +1567,7 @@ __device__ __forceinline__ void block_scan(int ncell, const unsigned int *__rest
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < ER_SCAN_CH; ++k) {
+            for (int k = 0; k < CH; ++k) {
                 if (b0 + k < ncell) start[b0 + k] = run;
                 run += v[k];
             }
@@ -1500,15 +1579,55 @@ __device__ __forceinline__ void block_scan(int ncell, const unsigned int *__rest
 }
 
 // both scans of the frame's sorts in one launch: block 0 the cells, block 1
-// the bricks
-__global__ void __launch_bounds__(1024) k_sort_scan(int ncell, const unsigned int *__restrict__ ccnt,
+// the bricks.  Four waves each: they run beside the plane DFTs, on whose CUs
+// a 1024-thread block waited up to 300 us for room.
+__global__ void __launch_bounds__(256) k_sort_scan(int ncell, const unsigned int *__restrict__ ccnt,
                                                     unsigned int *__restrict__ cstart, int nbrick,
                                                     const unsigned int *__restrict__ bcnt,
                                                     unsigned int *__restrict__ bstart)
 {
     __shared__ unsigned int wsum[16];
-    if (blockIdx.x == 0) block_scan(ncell, ccnt, cstart, wsum);
-    else block_scan(nbrick, bcnt, bstart, wsum);
+    if (blockIdx.x == 0) block_scan<32, 256>(ncell, ccnt, cstart, wsum);
+    else block_scan<32, 256>(nbrick, bcnt, bstart, wsum);
+}
+
+// Both sorts of a small frame (up to ER_SORT_ITEMS molecules and atoms on up
+// to ER_SORT_LDS cells and bricks) in one workgroup: counts and scans in LDS,
+// no device atomics and one launch instead of two (1000 waters: 8 us
+// against 9 + 5 us).
+#define ER_SORT_ITEMS 12288
+__global__ void __launch_bounds__(1024) k_sort_small(int nmol, const float4 *__restrict__ molref, FrameConst fc,
+                                                     SortGrid sg, int ncell, unsigned int *__restrict__ cstart,
+                                                     unsigned int *__restrict__ keyrank, float *__restrict__ rmolmax,
+                                                     int natom, const int4 *__restrict__ splg,
+                                                     unsigned int *__restrict__ bstart,
+                                                     unsigned int *__restrict__ akeyrank)
+{
+    extern __shared__ __align__(16) unsigned int lcnt[];  // [ncell] cells, then [nbrick] bricks
+    __shared__ unsigned int wsum[16];
+    const int tid = threadIdx.x, nb = sg.nbrick;
+    unsigned int *bc = lcnt + ncell;  // ncell is a multiple of 64
+    for (int b = tid; b < ncell + nb; b += 1024) lcnt[b] = 0u;
+    __syncthreads();
+    float R = 0.0f;
+    for (int t = tid; t < nmol; t += 1024) {
+        const float4 m = molref[t];
+        const unsigned int key = mol_cell(fc, sg, m);
+        keyrank[2 * t] = key;
+        keyrank[2 * t + 1] = atomicAdd(&lcnt[key], 1u);
+        R = fmaxf(R, m.w);
+    }
+    if (nb)
+        for (int a = tid; a < natom; a += 1024) {
+            const unsigned int key = atom_brick(sg, splg[a]);
+            akeyrank[2 * a] = key;
+            akeyrank[2 * a + 1] = atomicAdd(&bc[key], 1u);
+        }
+    for (int off = 32; off > 0; off >>= 1) R = fmaxf(R, __shfl_xor(R, off, 64));
+    if ((tid & 63) == 0) atomicMax(reinterpret_cast<unsigned int *>(rmolmax), __float_as_uint(R));
+    __syncthreads();
+    block_scan<8, 1024>(ncell, lcnt, cstart, wsum);
+    if (nb) block_scan<8, 1024>(nb, bc, bstart, wsum);
 }
 
 __global__ void k_cell_scatter(int nmol, const unsigned int *__restrict__ key_rank,
@@ -2453,7 +2572,7 @@ __device__ __forceinline__ void pair_candidates(const PairArgs &pa, const FrameC
         // cx + lo + dx lies in [-nreach, nc + nreach) with nreach < nc (or lo = 0):
         // one conditional wrap
         const int qx = wrap1(cx + lo + dx, pa.nc), qy = wrap1(cy + lo + dy, pa.nc), qz = wrap1(cz + lo + dz, pa.nc);
-        const unsigned int key = cell_key(qx, qy, qz);
+        const unsigned int key = cell_key(qx, qy, qz, pa.nc);
         const unsigned int p0 = cstart[key], p1 = cstart[key + 1];
         // the cell's molecules four at a time: indices, then centres
         for (unsigned int pb = p0; pb < p1; pb += 4) {
@@ -2626,7 +2745,7 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
         }
     __syncthreads();
     const int nclu = (pa.nslt + 7) >> 3;
-    if (in_lds && tid < nclu) clu[tid] = atom_sphere(fc, sx, tid * 8, min(tid * 8 + 8, pa.nslt));
+    if (in_lds && tid < nclu) clu[tid] = site_sphere(fc, [&](int a) { return sx[a]; }, tid * 8, min(tid * 8 + 8, pa.nslt), 0, 1);
     pair_candidates(pa, fc, ref, cut, part, skipmol, rmolmax[0], cstart, perm, molref, [&](int j) __attribute__((always_inline)) {
         if (atomicAdd(&ncand, 1) < ER_PAIR_CAP) {
             if (molbeg[j + 1] - molbeg[j] <= ER_PM_ATOMS) cand[atomicAdd(&nsmall, 1)] = j;
@@ -2940,12 +3059,6 @@ __global__ void __launch_bounds__(512) k_hist(HistArgs ha, int nslot, const Slot
         if (h && tile * NI + ii < ha.nchunk && ha.n_off + tile * NI + ii < live)
             atomicAdd(&Cnt[(size_t)(ha.n_off + tile * NI + ii) * ha.ermax + b], h);
     }
-}
-
-__global__ void k_zero_u32(size_t n, uint32_t *__restrict__ p)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0u;
 }
 
 // At the end of a run: if the halt key (thread 0) or the warning key (thread
