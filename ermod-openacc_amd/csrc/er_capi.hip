@@ -67,8 +67,8 @@ template <typename T> struct DBuf {
 
 }  // namespace
 
-// Scratch of er_run_noalloc: the split-K partial sums of edens/ecorr and the
-// weight kernel's block partials, in device memory that the library never
+// Scratch of er_run_noalloc: the split-K partial sums of edens/ecorr, in
+// device memory that the library never
 // allocates at run time.  Each GPU holds its own copy for the life of the
 // process.  In host code `scratch` names a host-side stand-in, not a device
 // address: kernels receive the per-device address that hipGetSymbolAddress
@@ -215,7 +215,6 @@ struct er_ctx {
 
     // energies / histograms
     DBuf<float> d_meshf, d_resself;
-    DBuf<double> d_wpart;  // k_weights block partials
     DBuf<unsigned short> d_blut;  // bin brackets per species (k_hist)
     DBuf<double> d_flpart;
     int nslice = 1;
@@ -232,7 +231,7 @@ struct er_ctx {
         int NI = NI_B;
         std::vector<int> order;    // slot ids in run order (few-site solutes first)
         std::vector<SlotDesc> desc;
-        int ntot = 0, nsite = 0, ndense = 0, pair_blocks = 0, nz = 0, wrow = 1;
+        int ntot = 0, nsite = 0, ndense = 0, pair_blocks = 0, nz = 0;
     } plan;
     DBuf<SlotDesc> d_sd;
     std::vector<SlotDesc> sd_up;   // what d_sd holds
@@ -1224,11 +1223,13 @@ template <int K2, int K3> static hipError_t launch_spec2d_k(er_ctx *c, int n_off
     if (sparse)
         hipLaunchKernelGGL((k_pme_spec2d<K2, K3, R1, R2, C1, C2, NT, true>), dim3(c->H, nch), dim3(NT), lds,
                            c->stream, nslot, c->d_sd.p, c->ord, c->K1, n_off, c->d_Ftab.p, c->d_insw.p,
-                           c->d_insg.p, c->d_engfac.p, c->d_tw2.p, c->d_tw3.p, c->d_tws.p, T, c->d_selfpart.p);
+                           c->d_insg.p, c->d_engfac.p, c->d_tw2.p, c->d_tw3.p, c->d_tws.p, T, c->d_selfpart.p,
+                           c->plan.ntot);
     else
         hipLaunchKernelGGL((k_pme_spec2d<K2, K3, R1, R2, C1, C2, NT, false>), dim3(c->H, nch), dim3(NT), lds,
                            c->stream, nslot, c->d_sd.p, c->ord, c->K1, n_off, c->d_Ftab.p, c->d_insw.p,
-                           c->d_insg.p, c->d_engfac.p, c->d_tw2.p, c->d_tw3.p, c->d_tws.p, T, c->d_selfpart.p);
+                           c->d_insg.p, c->d_engfac.p, c->d_tw2.p, c->d_tw3.p, c->d_tws.p, T, c->d_selfpart.p,
+                           c->plan.ntot);
     return hipGetLastError();
 }
 
@@ -1266,7 +1267,7 @@ static hipError_t launch_spec2d_mix(er_ctx *c, int n_off, int nch, int t_off, bo
                        (int)c->plan.desc.size(), c->d_sd.p, c->ord, c->K1, K2, K3, c->lp[1], c->lp[2],
                        div_magic(K2), div_magic(K3), c->d_rev[1].p, c->d_rev[2].p, (int)sparse, n_off, c->d_Ftab.p,
                        c->d_insw.p, c->d_insg.p, c->d_engfac.p, c->d_tw2.p, c->d_tw3.p, c->d_tws.p, T,
-                       c->d_selfpart.p);
+                       c->d_selfpart.p, c->plan.ntot);
     return hipGetLastError();
 }
 
@@ -1284,7 +1285,7 @@ static hipError_t launch_spec2d_gen(er_ctx *c, int n_off, int nch, int t_off, bo
     hipLaunchKernelGGL(k_pme_spec2d_gen, dim3(c->H, nch), dim3(ER_GEN_NT), lds, c->stream,
                        (int)c->plan.desc.size(), c->d_sd.p, c->ord, c->K1, c->K2, c->K3, (int)sparse, n_off,
                        c->d_Ftab.p, c->d_insw.p, c->d_insg.p, c->d_engfac.p, c->d_tw2.p, c->d_tw3.p, T,
-                       c->d_selfpart.p);
+                       c->d_selfpart.p, c->plan.ntot);
     return hipGetLastError();
 }
 
@@ -1487,8 +1488,9 @@ template <int NI> static hipError_t launch_hist(er_ctx *c, int n_off, int nch)
     // path's single-insertion tiles keep 256 (its per-thread partials are
     // reduced by one thread)
     const int NT = NI > 1 ? 512 : 256;
-    const size_t lds = (size_t)NT * sizeof(double) + (size_t)c->ermax * sizeof(float) +
-                       (size_t)NI * (c->ermax | 1) * sizeof(uint32_t) + (size_t)NT * 2 * sizeof(float) +
+    const size_t nred = (size_t)NT / 64 * NI;  // per-wave partials
+    const size_t lds = nred * sizeof(double) + (size_t)c->ermax * sizeof(float) +
+                       (size_t)NI * (c->ermax | 1) * sizeof(uint32_t) + nred * 2 * sizeof(float) +
                        (size_t)c->numslv * ER_LUT_N * sizeof(unsigned short);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
     if (lds > 65536)
@@ -1729,7 +1731,7 @@ static int build_plan(er_ctx *c, const std::vector<int> &todo, int mode)
             if ((c->slots[k].nslt > ER_SPARSE_SITES) == (pass == 1)) P.order.push_back(k);
     P.desc.assign(P.order.size(), SlotDesc{});
     long long ins = 0, site = 0, blk = 0;
-    int z = 0, wrow = 1;
+    int z = 0;
     P.ndense = 0;
     for (size_t i = 0; i < P.order.size(); ++i) {
         Slot &sl = c->slots[P.order[i]];
@@ -1763,7 +1765,6 @@ static int build_plan(er_ctx *c, const std::vector<int> &todo, int mode)
         site += (long long)nins * sl.nslt;
         blk += (long long)nins * d.pair_split;
         z += d.nks;
-        wrow = std::max(wrow, (nins + 255) / 256);
         if (sl.nslt <= ER_SPARSE_SITES) P.ndense = (int)ins;
     }
     if (ins >= (1ll << 30) || site >= (1ll << 30) || blk >= (1ll << 31) - 1)
@@ -1773,7 +1774,6 @@ static int build_plan(er_ctx *c, const std::vector<int> &todo, int mode)
     P.nsite = (int)site;
     P.pair_blocks = (int)blk;
     P.nz = z;
-    P.wrow = wrow;
     return ER_OK;
 }
 
@@ -1796,14 +1796,13 @@ static int upload_plan(er_ctx *c)
     return ER_OK;
 }
 
-// the split-K partials (ecorr, edens) and the weights' block partials of
-// the run: the context's buffers, or in an er_run_noalloc call consecutive
+// the split-K partials (ecorr, edens) of the run: the context's buffers, or in an er_run_noalloc call consecutive
 // ranges of the scratch array
 struct AccPartials {
-    double *part, *epart, *wpart;
+    double *part, *epart;
 };
 
-static void partial_sizes(const er_ctx *c, bool batched, size_t &npart, size_t &nepart, size_t &nwpart)
+static void partial_sizes(const er_ctx *c, bool batched, size_t &npart, size_t &nepart)
 {
     const auto &P = c->plan;
     int kper1, nks1;
@@ -1812,16 +1811,15 @@ static void partial_sizes(const er_ctx *c, bool batched, size_t &npart, size_t &
     const bool mfma = c->prm.corrcal == 1 && c->use_mfma;
     npart = mfma ? nz * c->ermax * c->ermax : 0;
     nepart = nz * c->ermax;
-    nwpart = batched ? (size_t)4 * P.desc.size() * P.wrow : 4;
 }
 
 static AccPartials acc_partials(er_ctx *c, bool batched)
 {
-    if (!c->noalloc) return {c->d_part.p, c->d_epart.p, c->d_wpart.p};
-    size_t np, ne, nw;
-    partial_sizes(c, batched, np, ne, nw);
+    if (!c->noalloc) return {c->d_part.p, c->d_epart.p};
+    size_t np, ne;
+    partial_sizes(c, batched, np, ne);
     double *p = c->scratch_dev;
-    return {p, p + np, p + np + ne};
+    return {p, p + np};
 }
 
 static int ensure_run_buffers(er_ctx *c, int chunk)
@@ -1838,17 +1836,16 @@ static int ensure_run_buffers(er_ctx *c, int chunk)
     } while (0)
     // the partial sums first: a run beyond the no-allocation scratch is refused outright
     {
-        size_t np, ne, nw;
-        partial_sizes(c, NI > 1, np, ne, nw);
+        size_t np, ne;
+        partial_sizes(c, NI > 1, np, ne);
         if (c->noalloc) {
-            if (np + ne + nw > ER_NOALLOC_SCRATCH_BYTES / sizeof(double))
+            if (np + ne > ER_NOALLOC_SCRATCH_BYTES / sizeof(double))
                 return fail(c, ER_E_UNSUPPORTED,
                             "er_run_noalloc: the run's partial sums (%d insertions, %d bins) need %zu bytes, above "
                             "the %zu-byte scratch (use er_run)",
-                            P.ntot, c->ermax, (np + ne + nw) * sizeof(double), (size_t)ER_NOALLOC_SCRATCH_BYTES);
+                            P.ntot, c->ermax, (np + ne) * sizeof(double), (size_t)ER_NOALLOC_SCRATCH_BYTES);
         } else {
             // at least the slices set_mesh sized, so small runs never shrink them
-            ER_WANT(c->d_wpart, nw);
             ER_WANT(c->d_epart, std::max(ne, (size_t)ER_KSLICES * c->ermax));
             if (np) ER_WANT(c->d_part, std::max(np, (size_t)ER_KSLICES * c->ermax * c->ermax));
         }
@@ -2025,16 +2022,14 @@ static hipError_t run_accumulate(er_ctx *c, AccRange ar)
         wa.screen = c->prm.screen;
         wa.qtot = c->qtot;
         wa.temp = c->prm.temp;
-        const int wrow = all ? P.wrow : std::max(1, (ar.nch + 255) / 256);
-        hipLaunchKernelGGL(k_weights_init, dim3(ns), dim3(64), 0, c->stream, wa, ar, sd, c->d_selfpart.p,
-                           c->d_selfreal.p, c->d_resself.p);
-        hipLaunchKernelGGL(k_weights, dim3(wrow, ns), dim3(256), 0, c->stream, wa, ar, sd, c->d_selfpart.p,
-                           c->d_selfreal.p, c->d_resself.p, c->d_u0cat.p, c->d_w.p,
+        int most = all ? 1 : ar.nch;
+        if (all)
+            for (const auto &d : P.desc) most = std::max(most, d.nins);
+        const int threads = std::min(1024, std::max(64, (most + 63) / 64 * 64));
+        hipLaunchKernelGGL(k_weights, dim3(ns), dim3(threads), 0, c->stream, wa, ar, sd, P.ntot, c->d_selfpart.p,
+                           c->d_selfreal.p, c->d_resself.p, c->d_u0cat.p, c->d_w.p, c->d_escrd.p,
                            soln ? c->d_flpart.p : (const double *)nullptr, soln ? c->d_flceng.p : (double *)nullptr,
-                           ap.wpart);
-        hipLaunchKernelGGL(k_weights_fin, dim3(ns), dim3(256), 0, c->stream, wa, ar, sd, wrow, ap.wpart,
-                           c->d_u0cat.p, c->d_w.p, c->d_escrd.p, soln ? c->d_flpart.p : (const double *)nullptr,
-                           soln ? c->d_flceng.p : (const double *)nullptr);
+                           P.NI, c->nummol, c->d_Ucat.p);
     }
     const int nz = all ? P.nz : (ar.nch + ar.kper - 1) / ar.kper;
     const bool mfma = c->prm.corrcal == 1 && c->use_mfma;
@@ -2155,9 +2150,6 @@ static int run_slots(er_ctx *c, const std::vector<int> &todo, int mode)
     }
     HIPCHK(c, join_atoms(c));  // a run without chunks still orders the next upload after the atom work
     if (c->capturing) ++c->capture_runs;
-    hipLaunchKernelGGL(k_halt_capture, dim3(nslot), dim3(64), 0, c->stream, sd, NI, c->nummol, c->d_Ucat.p,
-                       c->d_u0cat.p);
-    HIPCHK(c, hipGetLastError());
     for (int i = 0; i < nslot; ++i) {
         Slot &sl = c->slots[P.order[i]];
         sl.U_view = c->d_Ucat.p + (size_t)P.desc[i].ins_off * c->nummol;

@@ -834,7 +834,7 @@ __global__ void __launch_bounds__(NT) k_pme_spec2d(int nslot, const SlotDesc *__
                                                     const float *__restrict__ engfac,
                                                     const float2 *__restrict__ tw2, const float2 *__restrict__ tw3,
                                                     const float2 *__restrict__ tws, float2 *__restrict__ T,
-                                                    double *__restrict__ selfpart)
+                                                    double *__restrict__ selfpart, int ntot)
 {
     static_assert(R1 * R2 == K3 && C1 * C2 == K2, "line splits");
     constexpr int PS = K3 + 1;  // padded plane row stride
@@ -859,7 +859,7 @@ __global__ void __launch_bounds__(NT) k_pme_spec2d(int nslot, const SlotDesc *__
         // padding insertion: a zero plane and no self energy
         float2 *Tp = T + ((size_t)nl * H + m1) * (size_t)NE;
         for (int e = tid; e < NE; e += NT) Tp[e] = make_float2(0.f, 0.f);
-        if (tid == 0) selfpart[(size_t)n * H + m1] = 0.0;
+        if (tid == 0) selfpart[(size_t)m1 * ntot + n] = 0.0;
         return;
     }
     const int nslt = sd[ks].nslt;
@@ -1067,7 +1067,7 @@ __global__ void __launch_bounds__(NT) k_pme_spec2d(int nslot, const SlotDesc *__
     if (tid == 0) {
         double t = 0.0;
         for (int wv = 0; wv < NT / 64; ++wv) t += red[wv];
-        selfpart[(size_t)n * H + m1] = plane_weight(K1, m1) * t;
+        selfpart[(size_t)m1 * ntot + n] = plane_weight(K1, m1) * t;
     }
 }
 
@@ -1255,7 +1255,7 @@ __global__ void __launch_bounds__(ER_GEN_NT) k_pme_spec2d_gen(int nslot, const S
                                                               const float *__restrict__ engfac,
                                                               const float2 *__restrict__ tw2,
                                                               const float2 *__restrict__ tw3, float2 *__restrict__ T,
-                                                              double *__restrict__ selfpart)
+                                                              double *__restrict__ selfpart, int ntot)
 {
     constexpr int NT = ER_GEN_NT;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1272,7 +1272,7 @@ __global__ void __launch_bounds__(ER_GEN_NT) k_pme_spec2d_gen(int nslot, const S
     const int local = n - sd[ks].ins_off;
     if (local >= sd[ks].nins) {  // padding insertion: a zero plane and no self energy
         for (int e = tid; e < NE; e += NT) Tp[e] = make_float2(0.f, 0.f);
-        if (tid == 0) selfpart[(size_t)n * H + m1] = 0.0;
+        if (tid == 0) selfpart[(size_t)m1 * ntot + n] = 0.0;
         return;
     }
     const int nslt = sd[ks].nslt;
@@ -1350,7 +1350,7 @@ __global__ void __launch_bounds__(ER_GEN_NT) k_pme_spec2d_gen(int nslot, const S
     if (tid == 0) {
         double t = 0.0;
         for (int wv = 0; wv < NT / 64; ++wv) t += red[wv];
-        selfpart[(size_t)n * H + m1] = plane_weight(K1, m1) * t;
+        selfpart[(size_t)m1 * ntot + n] = plane_weight(K1, m1) * t;
     }
 }
 
@@ -2953,21 +2953,27 @@ __global__ void __launch_bounds__(512) k_hist(HistArgs ha, int nslot, const Slot
                                               uint32_t *__restrict__ Cnt, double *__restrict__ flpart)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    double *rsum = reinterpret_cast<double *>(smem);                 // [NT]
-    float *mesh = reinterpret_cast<float *>(rsum + blockDim.x);      // [ermax]
+    double *rsum = reinterpret_cast<double *>(smem);                 // [waves][NI]
+    float *mesh = reinterpret_cast<float *>(rsum + (blockDim.x >> 6) * NI);  // [ermax]
     // [NI][hs]: an odd row stride puts one bin of the NI rows (the lanes of a
     // wave hold NI insertions) in NI different banks
     const int hs = ha.ermax | 1;
     uint32_t *hist = reinterpret_cast<uint32_t *>(mesh + ha.ermax);
-    float *rmin = reinterpret_cast<float *>(hist + NI * hs);         // [NT]
-    float *rmax = rmin + blockDim.x;                                  // [NT]
-    unsigned short *blut = reinterpret_cast<unsigned short *>(rmax + blockDim.x);  // [numslv][ER_LUT_N]
+    float *rmin = reinterpret_cast<float *>(hist + NI * hs);         // [waves][NI]
+    float *rmax = rmin + (blockDim.x >> 6) * NI;                      // [waves][NI]
+    unsigned short *blut = reinterpret_cast<unsigned short *>(rmax + (blockDim.x >> 6) * NI);  // [numslv][ER_LUT_N]
 
     const int tid = threadIdx.x, NT = blockDim.x;
     const int tile = blockIdx.x, slice = blockIdx.y;
     for (int b = tid; b < ha.ermax; b += NT) mesh[b] = meshf[b];
     for (int b = tid; b < NI * hs; b += NT) hist[b] = 0u;
-    for (int b = tid; b < ha.numslv * ER_LUT_N; b += NT) blut[b] = lut[b];
+    {  // two brackets per load (the table is 256-byte aligned, blut 4-byte)
+        const int nl = ha.numslv * ER_LUT_N;
+        const unsigned int *l2 = reinterpret_cast<const unsigned int *>(lut);
+        unsigned int *d2 = reinterpret_cast<unsigned int *>(blut);
+        for (int b = tid; b < nl / 2; b += NT) d2[b] = l2[b];
+        if ((nl & 1) && tid == 0) blut[nl - 1] = lut[nl - 1];
+    }
     __syncthreads();
 
     const int i = tid % NI, jj = tid / NI, jstep = NT / NI;
@@ -3030,17 +3036,28 @@ __global__ void __launch_bounds__(512) k_hist(HistArgs ha, int nslot, const Slot
               }
             }
         }
-        rmin[tid] = lmin;
-        rmax[tid] = lmax;
-        rsum[tid] = lsum;
+        // over the wave's lanes of one insertion, then over the waves (a serial
+        // sum over the threads of an insertion cost 3 us per species)
+        const int lane = tid & 63, wave = tid >> 6, nw = NT >> 6;
+#pragma unroll
+        for (int off = NI; off < 64; off <<= 1) {
+            lmin = fminf(lmin, __shfl_xor(lmin, off, 64));
+            lmax = fmaxf(lmax, __shfl_xor(lmax, off, 64));
+            lsum += __shfl_xor(lsum, off, 64);
+        }
+        if (lane < NI) {
+            rmin[wave * NI + lane] = lmin;
+            rmax[wave * NI + lane] = lmax;
+            rsum[wave * NI + lane] = lsum;
+        }
         __syncthreads();
         if (tid < NI) {
             float mn = rmin[tid], mx = rmax[tid];
             double sm = rsum[tid];
-            for (int k = 1; k < jstep; ++k) {
-                mn = fminf(mn, rmin[tid + k * NI]);
-                mx = fmaxf(mx, rmax[tid + k * NI]);
-                sm += rsum[tid + k * NI];
+            for (int w = 1; w < nw; ++w) {
+                mn = fminf(mn, rmin[tid + w * NI]);
+                mx = fmaxf(mx, rmax[tid + w * NI]);
+                sm += rsum[tid + w * NI];
             }
             if (tile * NI + tid < ha.nchunk && ha.n_off + tile * NI + tid < live) {
                 if (mn <= mx) {
@@ -3053,33 +3070,15 @@ __global__ void __launch_bounds__(512) k_hist(HistArgs ha, int nslot, const Slot
         }
         __syncthreads();
     }
-    for (int f = tid; f < NI * ha.ermax; f += NT) {
-        const int ii = f / ha.ermax, b = f % ha.ermax;
-        const uint32_t h = hist[ii * hs + b];
-        if (h && tile * NI + ii < ha.nchunk && ha.n_off + tile * NI + ii < live)
-            atomicAdd(&Cnt[(size_t)(ha.n_off + tile * NI + ii) * ha.ermax + b], h);
+    // a wave per insertion row
+    for (int ii = tid >> 6; ii < NI; ii += NT >> 6) {
+        if (tile * NI + ii >= ha.nchunk || ha.n_off + tile * NI + ii >= live) continue;
+        uint32_t *row = Cnt + (size_t)(ha.n_off + tile * NI + ii) * ha.ermax;
+        for (int b = tid & 63; b < ha.ermax; b += 64) {
+            const uint32_t h = hist[ii * hs + b];
+            if (h) atomicAdd(&row[b], h);
+        }
     }
-}
-
-// At the end of a run: if the halt key (thread 0) or the warning key (thread
-// 1) belongs to this run and has not been captured yet, record the
-// offending energy while U / uvengy0 still hold it (cap[2t] = captured key,
-// cap[2t + 1] = the energy's bits).
-__global__ void k_halt_capture(const SlotDesc *__restrict__ sd, int NI, int nmol, const float *__restrict__ U,
-                               const float *__restrict__ u0)
-{
-    const int t = threadIdx.x;
-    if (t > 1) return;
-    const SlotDesc &d = sd[blockIdx.x];  // one block per solute of the run
-    const unsigned int seq = *d.seq;
-    unsigned long long *cap = d.halt;
-    const unsigned long long key = t == 0 ? *d.errkey : *d.warnkey;
-    if (key == ~0ull || (unsigned int)(key >> 42) != (seq & 0x3fffffu) || cap[2 * t] == key) return;
-    // the key holds the insertion within its solute
-    const int n = d.ins_off + (int)((key >> 21) & 0x1fffffu), jp1 = (int)(key & 0x1fffffu);
-    const float v = jp1 == 0 ? u0[n] : U[((size_t)(n / NI) * nmol + (jp1 - 1)) * NI + (n % NI)];
-    cap[2 * t] = key;
-    cap[2 * t + 1] = (unsigned long long)__float_as_uint(v);
 }
 
 // ---------------------------------------------------------------------------
@@ -3097,8 +3096,7 @@ struct WeightArgs {
 };
 
 // The insertions an accumulation covers.  nch < 0: every solute of the run,
-// solute = blockIdx.y (k_weights) / blockIdx.x (init, fin) / the slice's
-// solute (k_ecorr), each over all its insertions.  nch >= 0: solute `slot`
+// solute = blockIdx.x (k_weights) / the slice's solute (k_ecorr), each over all its insertions.  nch >= 0: solute `slot`
 // only, its insertions [rel, rel + nch) (the plain path), kper insertions
 // per ecorr slice.
 struct AccRange {
@@ -3120,73 +3118,66 @@ __device__ __forceinline__ void acc_span(const AccRange &r, const SlotDesc *__re
     }
 }
 
-// uvengy0 of insertion n: uvrecp (FP64 half-plane partials) + pairep +
-// residual, in the reference's real arithmetic
-__device__ __forceinline__ float weights_uv0(const WeightArgs &wa, const double *__restrict__ selfpart,
+// uvengy0 of insertion n: uvrecp (FP64 half-plane partials, [m1][insertion])
+// + pairep + residual, in the reference's real arithmetic
+__device__ __forceinline__ float weights_uv0(const WeightArgs &wa, const double *__restrict__ selfpart, int ntot,
                                              const float *__restrict__ resself, int n, float real)
 {
     double rec = 0.0;
-    for (int m = 0; m < wa.H; ++m) rec += selfpart[(size_t)n * wa.H + m];
+#pragma unroll 8
+    for (int m = 0; m < wa.H; ++m) rec += selfpart[(size_t)m * ntot + n];
     return (float)rec + real + resself[n];
 }
 
-// first run of a block: the rigid solute's real self term and voffset (one
-// block per solute)
-__global__ void k_weights_init(WeightArgs wa, AccRange ar, const SlotDesc *__restrict__ sd,
-                               const double *__restrict__ selfpart, const float *__restrict__ selfreal,
-                               const float *__restrict__ resself)
+// One workgroup per solute, a thread per insertion in turn: on the first run
+// of a block the rigid solute's real self term and voffset; uvengy0; the weight
+// engnmfc (engproc.F90:858-912); flceng; the scalar accumulators; the
+// sequential parts in n as the reference adds them (self-energy distribution,
+// slnuv); and last the halt capture.  Latency-bound (a few KB per solute):
+// one launch instead of four (5 + 17 + 5 + 4 us at 1000 insertions, WGT us
+// together), with the plane partials read across the insertions.
+__global__ void __launch_bounds__(1024) k_weights(WeightArgs wa, AccRange ar, const SlotDesc *__restrict__ sd,
+                                                  int ntot, const double *__restrict__ selfpart,
+                                                  const float *__restrict__ selfreal,
+                                                  const float *__restrict__ resself, float *u0, double *wout,
+                                                  const double *__restrict__ escrd,
+                                                  const double *__restrict__ flpart, double *flceng, int NI, int nmol,
+                                                  const float *__restrict__ U)
 {
-    if (threadIdx.x != 0) return;
+    __shared__ double r_w[16], r_t[16];
+    __shared__ float r_mn[16], r_mx[16];
+    __shared__ float first_u;
+    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wave = tid >> 6, nw = NT >> 6;
     int k, n_off, nchunk;
     acc_span(ar, sd, blockIdx.x, k, n_off, nchunk);
+    double *__restrict__ state = sd[k].state;
     int *flags = sd[k].flags;
     float *fstate = sd[k].fstate;
-    if (wa.rigid && !flags[1]) {
-        fstate[0] = selfreal[n_off];
-        flags[1] = 1;
-    }
-    if (wa.wgtslf && !flags[0]) {
-        const float real0 = wa.rigid ? fstate[0] : selfreal[n_off];
-        sd[k].state[3] = (double)weights_uv0(wa, selfpart, resself, n_off, real0);
-        flags[0] = 1;
-    }
-}
-
-// per insertion (one thread each): uvengy0, the weight engnmfc
-// (engproc.F90:858-912), flceng; per block: fixed-order tree partials of
-// sum w, sum w_tot and the min/max of uvengy0 into wpart[block][4]
-__global__ void __launch_bounds__(256) k_weights(WeightArgs wa, AccRange ar, const SlotDesc *__restrict__ sd,
-                                                 const double *__restrict__ selfpart,
-                                                 const float *__restrict__ selfreal,
-                                                 const float *__restrict__ resself,
-                                                 float *__restrict__ u0, double *__restrict__ wout,
-                                                 const double *__restrict__ flpart, double *__restrict__ flceng,
-                                                 double *__restrict__ wpart)
-{
-    __shared__ double r_w[256], r_t[256];
-    __shared__ float r_mn[256], r_mx[256];
-    const int tid = threadIdx.x, NT = blockDim.x;
-    int k, n_off, nchunk;
-    acc_span(ar, sd, blockIdx.y, k, n_off, nchunk);  // grid.y: the run's solutes
-    const double voffset = gptr(sd[k].state)[3];
-    const float usreal = gptr(sd[k].fstate)[0];
+    const bool have_real = flags[1] != 0, have_off = flags[0] != 0;
+    const float usreal = have_real ? fstate[0] : selfreal[n_off];
+    const double voff0 = state[3];
     const __attribute__((address_space(1))) float *wslt = sd[k].wslt ? gptr(sd[k].wslt) : nullptr;
-    double sw = 0.0, st = 0.0;
+    const int base = sd[k].ins_off;  // halt keys hold the insertion within its solute
     float mn = 3.402823466e38f, mx = -3.402823466e38f;
-    const int nl = blockIdx.x * NT + tid;
-    if (nl < nchunk) {
+    for (int nl = tid; nl < nchunk; nl += NT) {
         const int n = n_off + nl;
-        const float real = wa.rigid ? usreal : selfreal[n];
-        const float u = weights_uv0(wa, selfpart, resself, n, real);
+        const float u = weights_uv0(wa, selfpart, ntot, resself, n, wa.rigid ? usreal : selfreal[n]);
         u0[n] = u;
-        mn = u;
-        mx = u;
+        mn = fminf(mn, u);
+        mx = fmaxf(mx, u);
+        if (nl == 0) first_u = u;
+    }
+    __syncthreads();
+    const double voffset = wa.wgtslf && !have_off ? (double)first_u : voff0;
+    double sw = 0.0, st = 0.0;
+    for (int nl = tid; nl < nchunk; nl += NT) {
+        const int n = n_off + nl;
         double engnmfc = 1.0;
         if (wa.wgtslf) {
-            const float factor = (float)((double)u - voffset);
+            const float factor = (float)((double)u0[n] - voffset);
             engnmfc = (wa.slttype == 1) ? exp((double)factor / wa.temp) : exp(-(double)factor / wa.temp);
         }
-        float tw = wa.w_sys * (wslt ? wslt[n - sd[k].ins_off] : 1.0f);
+        float tw = wa.w_sys * (wslt ? wslt[n - base] : 1.0f);
         if (wa.estype == 2) {  // volcorrect (engproc.F90:1022-1038)
             tw = tw * wa.volume;
             if (!wa.bare) {
@@ -3196,80 +3187,59 @@ __global__ void __launch_bounds__(256) k_weights(WeightArgs wa, AccRange ar, con
         }
         engnmfc *= (double)tw;
         wout[n] = engnmfc;
-        sw = engnmfc;
-        st = (double)tw;
-        if (flpart) {  // flceng(sp, n): slices summed in a fixed order
-            for (int sp = 0; sp < wa.numslv; ++sp) {
-                double s = 0.0;
-                for (int sl = 0; sl < wa.nslice; ++sl) s += flpart[((size_t)n * wa.nslice + sl) * wa.numslv + sp];
-                flceng[(size_t)n * wa.numslv + sp] = s;
-            }
-        }
+        sw += engnmfc;
+        st += (double)tw;
     }
-    r_w[tid] = sw;
-    r_t[tid] = st;
-    r_mn[tid] = mn;
-    r_mx[tid] = mx;
+    // flceng(sp, n): one wave per (insertion, species), the slices over its lanes
+    if (flpart)
+        for (int t = wave; t < nchunk * wa.numslv; t += nw) {
+            const int n = n_off + t / wa.numslv, sp = t % wa.numslv;
+            double f = 0.0;
+            for (int sl = lane; sl < wa.nslice; sl += 64) f += flpart[((size_t)n * wa.nslice + sl) * wa.numslv + sp];
+            for (int off = 32; off > 0; off >>= 1) f += __shfl_xor(f, off, 64);
+            if (lane == 0) flceng[(size_t)n * wa.numslv + sp] = f;
+        }
+    for (int off = 32; off > 0; off >>= 1) {
+        sw += __shfl_xor(sw, off, 64);
+        st += __shfl_xor(st, off, 64);
+        mn = fminf(mn, __shfl_xor(mn, off, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    }
+    if (lane == 0) {
+        r_w[wave] = sw;
+        r_t[wave] = st;
+        r_mn[wave] = mn;
+        r_mx[wave] = mx;
+    }
     __syncthreads();
-    for (int s = NT / 2; s > 0; s >>= 1) {
-        if (tid < s) {
-            r_w[tid] += r_w[tid + s];
-            r_t[tid] += r_t[tid + s];
-            r_mn[tid] = fminf(r_mn[tid], r_mn[tid + s]);
-            r_mx[tid] = fmaxf(r_mx[tid], r_mx[tid + s]);
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {  // each solute's partials in its own row of gridDim.x blocks
-        double *wp = wpart + 4 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x);
-        wp[0] = r_w[0];
-        wp[1] = r_t[0];
-        wp[2] = (double)r_mn[0];
-        wp[3] = (double)r_mx[0];
-    }
-}
-
-// the block partials in block order, then the sequential parts: the
-// self-energy distribution and slnuv, in n as the reference adds them
-__global__ void __launch_bounds__(256) k_weights_fin(WeightArgs wa, AccRange ar, const SlotDesc *__restrict__ sd,
-                                                     int wrow, const double *__restrict__ wpart_all,
-                                                     const float *__restrict__ u0,
-                                                     const double *__restrict__ wout,
-                                                     const double *__restrict__ escrd,
-                                                     const double *__restrict__ flpart,
-                                                     const double *__restrict__ flceng)
-{
-    // one block per solute; wrow = k_weights' blocks per solute row of wpart
-    const int tid = threadIdx.x;
-    int k, n_off, nchunk;
-    acc_span(ar, sd, blockIdx.x, k, n_off, nchunk);
-    const int nblk = max(1, (nchunk + 255) / 256);
-    const double *__restrict__ wpart = wpart_all + 4 * (size_t)blockIdx.x * wrow;
-    double *__restrict__ state = sd[k].state;
-    double *__restrict__ eself = sd[k].eself;
-    double *__restrict__ slnuv = sd[k].slnuv;
-    unsigned int *__restrict__ minmax = sd[k].minmax;
     const unsigned int seq = *sd[k].seq;
-    const int base = sd[k].ins_off;  // halt keys hold the insertion within its solute
     if (tid == 0) {
-        double sw = 0.0, st = 0.0;
-        float mn = 3.402823466e38f, mx = -3.402823466e38f;
-        for (int b = 0; b < nblk; ++b) {
-            sw += wpart[4 * b + 0];
-            st += wpart[4 * b + 1];
-            mn = fminf(mn, (float)wpart[4 * b + 2]);
-            mx = fmaxf(mx, (float)wpart[4 * b + 3]);
+        for (int w = 1; w < nw; ++w) {
+            sw += r_w[w];
+            st += r_t[w];
+            mn = fminf(mn, r_mn[w]);
+            mx = fmaxf(mx, r_mx[w]);
         }
         state[0] += sw;
         state[1] += (double)nchunk;
         state[2] += st;
+        if (wa.wgtslf && !have_off) {
+            state[3] = voffset;
+            flags[0] = 1;
+        }
+        if (wa.rigid && !have_real) {
+            fstate[0] = usreal;
+            flags[1] = 1;
+        }
         // solute self-energy extremes (engproc.F90:914-915)
+        unsigned int *minmax = sd[k].minmax;
         if (nchunk > 0) {
             gatomic_min(&minmax[0], f2ord(mn));
             gatomic_max(&minmax[1], f2ord(mx));
         }
         // self-energy distribution, sequential in n as the reference adds it
         if (wa.selfcal) {
+            double *eself = sd[k].eself;
             for (int nl = 0; nl < nchunk; ++nl) {
                 const int n = n_off + nl;
                 const float u = u0[n];
@@ -3283,16 +3253,33 @@ __global__ void __launch_bounds__(256) k_weights_fin(WeightArgs wa, AccRange ar,
                 if (lo == wa.esmax && u < 1.0e3f) gatomic_min(sd[k].warnkey, halt_key(seq, n - base, 0));
                 gptr(eself)[max(lo, 1) - 1] += wout[n];
             }
+            __threadfence();
         }
     }
     // slnuv += flceng * engnmfc (engproc.F90:939-941), sequential in n
     if (flpart && tid < wa.numslv) {
+        double *slnuv = sd[k].slnuv;
         double s = slnuv[tid];
         for (int nl = 0; nl < nchunk; ++nl) {
             const int n = n_off + nl;
             s += flceng[(size_t)n * wa.numslv + tid] * wout[n];
         }
         slnuv[tid] = s;
+    }
+    __syncthreads();
+    // If the halt key (thread 0) or the warning key (thread 1) belongs to this
+    // run and has not been captured yet, record the offending energy while U /
+    // uvengy0 still hold it (cap[2t] = captured key, cap[2t + 1] = the energy's bits).
+    if (tid <= 1) {
+        unsigned long long *cap = sd[k].halt;
+        const unsigned long long key = __hip_atomic_load(gptr(tid == 0 ? sd[k].errkey : sd[k].warnkey),
+                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (key == ~0ull || (unsigned int)(key >> 42) != (seq & 0x3fffffu) || cap[2 * tid] == key) return;
+        // the key holds the insertion within its solute
+        const int n = base + (int)((key >> 21) & 0x1fffffu), jp1 = (int)(key & 0x1fffffu);
+        const float v = jp1 == 0 ? u0[n] : U[((size_t)(n / NI) * nmol + (jp1 - 1)) * NI + (n % NI)];
+        cap[2 * tid] = key;
+        cap[2 * tid + 1] = (unsigned long long)__float_as_uint(v);
     }
 }
 

@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(512) k_pme_spec2d_mix(int nslot, const SlotDes
                                                         const float2 *__restrict__ tw2,
                                                         const float2 *__restrict__ tw3,
                                                         const float2 *__restrict__ tws, float2 *__restrict__ T,
-                                                        double *__restrict__ selfpart)
+                                                        double *__restrict__ selfpart, int ntot)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int PS = K3 | 1, NE = K2 * K3, H = K1 / 2 + 1;
@@ -229,7 +229,7 @@ __global__ void __launch_bounds__(512) k_pme_spec2d_mix(int nslot, const SlotDes
     const int local = n - sd[ks].ins_off;
     if (local >= sd[ks].nins) {  // padding insertion: a zero plane and no self energy
         for (int e = tid; e < NE; e += NT) Tp[e] = make_float2(0.f, 0.f);
-        if (tid == 0) selfpart[(size_t)n * H + m1] = 0.0;
+        if (tid == 0) selfpart[(size_t)m1 * ntot + n] = 0.0;
         return;
     }
     const int nslt = sd[ks].nslt;
@@ -312,7 +312,7 @@ __global__ void __launch_bounds__(512) k_pme_spec2d_mix(int nslot, const SlotDes
     if (tid == 0) {
         double t = 0.0;
         for (int wv = 0; wv < (NT >> 6); ++wv) t += red[wv];
-        selfpart[(size_t)n * H + m1] = plane_weight(K1, m1) * t;
+        selfpart[(size_t)m1 * ntot + n] = plane_weight(K1, m1) * t;
     }
 }
 
