@@ -65,6 +65,32 @@ template <typename T> struct DBuf {
     }
 };
 
+// page-locked host memory of one context: kernels write it, copies to and from
+// the device run beside the host
+template <typename T> struct HBuf {
+    T *p = nullptr;
+    size_t n = 0;
+    HBuf() = default;
+    HBuf(const HBuf &) = delete;
+    HBuf &operator=(const HBuf &) = delete;
+    ~HBuf() { release(); }
+    hipError_t ensure(size_t count)
+    {
+        if (count <= n && p) return hipSuccess;
+        release();
+        const hipError_t e = hipHostMalloc((void **)&p, std::max<size_t>(count, 1) * sizeof(T), hipHostMallocDefault);
+        if (e == hipSuccess) n = count;
+        else p = nullptr;
+        return e;
+    }
+    void release()
+    {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        n = 0;
+    }
+};
+
 }  // namespace
 
 // Scratch of er_run_noalloc: the split-K partial sums of edens/ecorr, in
@@ -255,6 +281,21 @@ struct er_ctx {
     double *scratch_dev = nullptr;
     bool noalloc = false;
 
+    // Host side of the calls' copies, in page-locked memory (a copy from
+    // pageable memory holds the caller for the whole transfer and one into it
+    // for 13 us however small): uploads go through a ring of buffers, each
+    // reused once its copy has run; the halts and flceng are written by the
+    // kernels themselves; results leave through h_res and, in ER_EC_CHUNK
+    // pieces, ecorr through h_ec.
+    HBuf<char> h_up[4];
+    hipEvent_t ev_up[4] = {};
+    bool up_busy[4] = {};
+    int up_next = 0;
+    HBuf<unsigned long long> h_halt;  // [slots][6]
+    HBuf<double> h_flceng, h_res;
+    HBuf<char> h_ec;
+    hipEvent_t ev_ec[4] = {};
+
     // diagnostics: event pairs recorded around launches while profiling
     bool prof = false;
     struct ProfRec { int kind; hipEvent_t a, b; };
@@ -288,6 +329,34 @@ static int fail(er_ctx *c, int code, const char *fmt, ...)
         c->errmsg = buf;
     }
     return code;
+}
+
+static hipError_t lazy_event(hipEvent_t &e)
+{
+    return e ? hipSuccess : hipEventCreateWithFlags(&e, hipEventDisableTiming);
+}
+
+// host bytes to the device in the stream's order; the caller's array is free on
+// return.  Beyond ER_UP_MAX the copy is made synchronously instead.
+#define ER_UP_MAX ((size_t)32 << 20)
+static hipError_t upload(er_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    hipError_t e;
+    if (bytes > ER_UP_MAX) {
+        if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return e;
+        return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+    }
+    const int k = c->up_next;
+    c->up_next = (k + 1) & 3;
+    if ((e = lazy_event(c->ev_up[k])) != hipSuccess) return e;
+    if (c->up_busy[k] && (e = hipEventSynchronize(c->ev_up[k])) != hipSuccess) return e;
+    c->up_busy[k] = false;
+    if ((e = c->h_up[k].ensure(bytes)) != hipSuccess) return e;
+    std::memcpy(c->h_up[k].p, src, bytes);
+    if ((e = hipMemcpyAsync(dst, c->h_up[k].p, bytes, hipMemcpyHostToDevice, c->stream)) != hipSuccess) return e;
+    if ((e = hipEventRecord(c->ev_up[k], c->stream)) != hipSuccess) return e;
+    c->up_busy[k] = true;
+    return hipSuccess;
 }
 
 static hipEvent_t prof_event(er_ctx *c)
@@ -495,6 +564,16 @@ static int slot_state_init(er_ctx *c, Slot &sl)
     return ER_OK;
 }
 
+// the host's view of the halts: none (no run is in flight)
+static hipError_t halt_mirror_init(er_ctx *c)
+{
+    const size_t n = 6 * c->slots.size();
+    const hipError_t e = c->h_halt.ensure(n);
+    if (e != hipSuccess) return e;
+    for (size_t k = 0; k < n; ++k) c->h_halt.p[k] = ~0ull;
+    return hipSuccess;
+}
+
 // mesh-sized per-slot accumulators (contents cleared by er_clear)
 static int slot_acc_alloc(er_ctx *c, Slot &sl)
 {
@@ -504,15 +583,26 @@ static int slot_acc_alloc(er_ctx *c, Slot &sl)
     return ER_OK;
 }
 
-static int slot_clear(er_ctx *c, Slot &sl)
+// the block accumulators of every slot, in the stream's order
+static int clear_slots(er_ctx *c)
 {
-    hipStream_t s = c->stream;
-    HIPCHK(c, hipMemsetAsync(sl.d_edens.p, 0, c->ermax * sizeof(double), s));
-    HIPCHK(c, hipMemsetAsync(sl.d_ecorr.p, 0, (size_t)c->ermax * c->ermax * sizeof(double), s));
-    HIPCHK(c, hipMemsetAsync(sl.d_eself.p, 0, std::max(1, c->esmax) * sizeof(double), s));
-    HIPCHK(c, hipMemsetAsync(sl.d_slnuv.p, 0, c->numslv * sizeof(double), s));
-    // engnorm, engsmpl, avslf (voffset survives, engproc.F90:336-338)
-    HIPCHK(c, hipMemsetAsync(sl.d_state.p, 0, 3 * sizeof(double), s));
+    for (size_t k0 = 0; k0 < c->slots.size(); k0 += ER_CLEAR_SLOTS) {
+        ClearArgs ca{};
+        const size_t n = std::min<size_t>(ER_CLEAR_SLOTS, c->slots.size() - k0);
+        for (size_t k = 0; k < n; ++k) {
+            Slot &sl = c->slots[k0 + k];
+            ca.edens[k] = sl.d_edens.p;
+            ca.ecorr[k] = sl.d_ecorr.p;
+            ca.eself[k] = sl.d_eself.p;
+            ca.slnuv[k] = sl.d_slnuv.p;
+            ca.state[k] = sl.d_state.p;
+        }
+        const size_t words = std::max<size_t>((size_t)c->ermax * c->ermax, (size_t)c->numslv);
+        const unsigned blocks = (unsigned)std::min<size_t>(1024, (words + 1023) / 1024);
+        hipLaunchKernelGGL(k_clear, dim3(blocks, (unsigned)n), dim3(256), 0, c->stream, ca, c->ermax,
+                           std::max(1, c->esmax), c->numslv);
+        HIPCHK(c, hipGetLastError());
+    }
     return ER_OK;
 }
 
@@ -726,6 +816,7 @@ extern "C" int er_create(const er_topology *topo, const er_params *prm, er_ctx *
     {
         const int rc = slot_state_init(c, c->slots[0]);
         if (rc) return bad(rc);
+        HIPCHK(c, halt_mirror_init(c));
     }
     // Accumulator layout of the FP64 MFMA: each output register of a known
     // product names its own (row, col); use the MFMA path only if the
@@ -890,11 +981,13 @@ extern "C" int er_set_solutes(er_ctx *c, int32_t nsolute, const int32_t *nsite, 
         int rc = set_slot_solute(c, sl, nsite[k], ljtype + off, charge + off);
         if (!rc) rc = slot_state_init(c, sl);
         if (!rc && c->have_mesh) rc = slot_acc_alloc(c, sl);
-        if (!rc && c->have_mesh) rc = slot_clear(c, sl);
         if (rc) return rc;
         sl.have_ins = false;
         off += (size_t)nsite[k];
     }
+    HIPCHK(c, halt_mirror_init(c));
+    const int rc = c->have_mesh ? clear_slots(c) : ER_OK;
+    if (rc) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return ER_OK;
 }
@@ -929,6 +1022,7 @@ extern "C" int er_set_solute_molecules(er_ctx *c, int32_t nslt, const int32_t *t
     c->S().nslt = ns;
     HIPCHK(c, hipStreamSynchronize(c->stream));  // a run in flight may still read the list
     HIPCHK(c, c->d_tag.ensure(nslt));
+    HIPCHK(c, c->h_flceng.ensure((size_t)nslt * c->numslv));
     HIPCHK(c, hipMemcpy(c->d_tag.p, c->tagslt.data(), nslt * sizeof(int), hipMemcpyHostToDevice));
     return ER_OK;
 }
@@ -1115,9 +1209,8 @@ extern "C" int er_set_frame(er_ctx *c, const float *sitepos, const float *cell, 
     if (!sitepos || !cell) return fail(c, ER_E_ARG, "er_set_frame: null argument");
     int rc = frame_cell(c, cell);
     if (rc) return rc;
-    // the previous run may still read the buffer
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    HIPCHK(c, hipMemcpy(c->d_sitepos_own.p, sitepos, (size_t)3 * c->numatm * sizeof(float), hipMemcpyHostToDevice));
+    // in the stream's order: the previous run has read the buffer by then
+    HIPCHK(c, upload(c, c->d_sitepos_own.p, sitepos, (size_t)3 * c->numatm * sizeof(float)));
     c->d_sitepos = c->d_sitepos_own.p;
     c->w_sys = stat_weight_system;
     c->have_frame = true;
@@ -1145,18 +1238,18 @@ static int ins_common(er_ctx *c, int32_t nins, const float *wslt, bool copies)
     if (nins <= 0) return fail(c, ER_E_ARG, "nins must be positive");
     if (c->capturing && (copies || wslt))
         return fail(c, ER_E_STATE, "a recorded graph takes er_set_insertions_device without stat_weight_solute");
-    // a run still in flight may read the buffers about to be overwritten
-    if (copies || wslt) HIPCHK(c, hipStreamSynchronize(c->stream));
     if (c->capturing && c->S().d_wslt.n < (size_t)nins)
         return fail(c, ER_E_STATE, "er_graph_begin: run these insertions once before recording");
     c->S().nins = nins;
     {
         const float *before = c->S().d_wslt.p;
+        // a run still in flight may read a buffer about to be replaced
+        if ((size_t)nins > c->S().d_wslt.n && !c->capturing) HIPCHK(c, hipStreamSynchronize(c->stream));
         HIPCHK(c, c->S().d_wslt.ensure(nins));
         if (c->S().d_wslt.p != before) ++c->alloc_gen;
     }
     c->S().wslt_given = wslt != nullptr;
-    if (wslt) HIPCHK(c, hipMemcpy(c->S().d_wslt.p, wslt, nins * sizeof(float), hipMemcpyHostToDevice));
+    if (wslt) HIPCHK(c, upload(c, c->S().d_wslt.p, wslt, nins * sizeof(float)));
     c->S().have_ins = true;
     return ER_OK;
 }
@@ -1168,8 +1261,9 @@ extern "C" int er_set_insertions(er_ctx *c, int32_t nins, const float *sltpos, c
     int rc = ins_common(c, nins, stat_weight_solute, true);
     if (rc) return rc;
     const size_t n = (size_t)3 * c->S().nslt * nins;
-    HIPCHK(c, c->S().d_sltpos_own.ensure(n));  // read only by the runs' copy of the coordinates
-    HIPCHK(c, hipMemcpy(c->S().d_sltpos_own.p, sltpos, n * sizeof(float), hipMemcpyHostToDevice));
+    if (n > c->S().d_sltpos_own.n) HIPCHK(c, hipStreamSynchronize(c->stream));  // a run in flight may read it
+    HIPCHK(c, c->S().d_sltpos_own.ensure(n));
+    HIPCHK(c, upload(c, c->S().d_sltpos_own.p, sltpos, n * sizeof(float)));
     c->S().d_sltpos = c->S().d_sltpos_own.p;
     return ER_OK;
 }
@@ -1761,6 +1855,7 @@ static int build_plan(er_ctx *c, const std::vector<int> &todo, int mode)
         d.errkey = sl.d_errkey.p;
         d.warnkey = sl.d_warnkey.p;
         d.halt = sl.d_halt.p;
+        d.hhalt = c->h_halt.p + 6 * (size_t)P.order[i];
         ins += (nins + P.NI - 1) / P.NI * P.NI;
         site += (long long)nins * sl.nslt;
         blk += (long long)nins * d.pair_split;
@@ -2029,7 +2124,7 @@ static hipError_t run_accumulate(er_ctx *c, AccRange ar)
         hipLaunchKernelGGL(k_weights, dim3(ns), dim3(threads), 0, c->stream, wa, ar, sd, P.ntot, c->d_selfpart.p,
                            c->d_selfreal.p, c->d_resself.p, c->d_u0cat.p, c->d_w.p, c->d_escrd.p,
                            soln ? c->d_flpart.p : (const double *)nullptr, soln ? c->d_flceng.p : (double *)nullptr,
-                           P.NI, c->nummol, c->d_Ucat.p);
+                           c->h_flceng.p, P.NI, c->nummol, c->d_Ucat.p);
     }
     const int nz = all ? P.nz : (ar.nch + ar.kper - 1) / ar.kper;
     const bool mfma = c->prm.corrcal == 1 && c->use_mfma;
@@ -2221,8 +2316,7 @@ extern "C" int er_run_noalloc(er_ctx *c, int32_t mode)
 static void decode_halt(er_ctx *c, unsigned long long key, bool warn)
 {
     const int jp1 = (int)(key & 0x1fffffu);
-    unsigned long long cap[4] = {~0ull, 0ull, ~0ull, 0ull};
-    (void)hipMemcpy(cap, c->S().d_halt.p, sizeof cap, hipMemcpyDeviceToHost);
+    const unsigned long long *cap = c->h_halt.p + 6 * (size_t)c->cur + 2;
     const int o = warn ? 2 : 0;
     float v = 0.f;
     if (cap[o] == key) {
@@ -2261,9 +2355,7 @@ extern "C" int er_sync(er_ctx *c)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const int keep = c->cur;
     for (int k = 0; k < (int)c->slots.size(); ++k) {
-        unsigned long long key = ~0ull, wkey = ~0ull;
-        HIPCHK(c, hipMemcpy(&key, c->slots[k].d_errkey.p, sizeof key, hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(&wkey, c->slots[k].d_warnkey.p, sizeof wkey, hipMemcpyDeviceToHost));
+        unsigned long long key = c->h_halt.p[6 * k], wkey = c->h_halt.p[6 * k + 1];
         // getiduv tests the halt conditions before the warning, so at equal
         // keys (one energy) the halt is met first
         const bool warn = !c->prm.force_calculation && wkey < key;
@@ -2316,27 +2408,55 @@ extern "C" int er_fetch(er_ctx *c, double *edens, double *ecorr, double *eself, 
     if (!c) return ER_E_ARG;
     ER_NO_CAPTURE(c, "er_fetch");
     if (!c->have_mesh) return fail(c, ER_E_STATE, "er_fetch: no mesh");
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (edens) HIPCHK(c, hipMemcpy(edens, c->S().d_edens.p, c->ermax * sizeof(double), hipMemcpyDeviceToHost));
-    if (ecorr)
-        HIPCHK(c, hipMemcpy(ecorr, c->S().d_ecorr.p, (size_t)c->ermax * c->ermax * sizeof(double), hipMemcpyDeviceToHost));
-    if (eself && c->esmax > 0) HIPCHK(c, hipMemcpy(eself, c->S().d_eself.p, c->esmax * sizeof(double), hipMemcpyDeviceToHost));
-    if (scal) HIPCHK(c, hipMemcpy(scal, c->S().d_state.p, 4 * sizeof(double), hipMemcpyDeviceToHost));
-    if (minuv || maxuv) {
-        std::vector<unsigned int> mm(2 * (size_t)(c->numslv + 1));
-        HIPCHK(c, hipMemcpy(mm.data(), c->S().d_minmax.p, mm.size() * sizeof(unsigned int), hipMemcpyDeviceToHost));
-        auto unord = [](unsigned int u) {
-            u = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
-            float f;
-            std::memcpy(&f, &u, 4);
-            return f;
+    Slot &sl = c->S();
+    const int es = std::max(1, c->esmax), ns = c->numslv;
+    HIPCHK(c, c->h_res.ensure((size_t)c->ermax + es + 4 + ns + (ns + 1)));
+    hipLaunchKernelGGL(k_fetch, dim3(1), dim3(1024), 0, c->stream, c->ermax, es, ns, sl.d_edens.p, sl.d_eself.p,
+                       sl.d_state.p, sl.d_slnuv.p, sl.d_minmax.p, c->h_res.p);
+    HIPCHK(c, hipGetLastError());
+    if (ecorr) {
+        // ecorr in pieces through four page-locked buffers, the copies of the
+        // next pieces under the host's copy of one (600 bins: 190 us against
+        // 232 for a copy straight into fresh pageable memory)
+        const size_t total = (size_t)c->ermax * c->ermax * sizeof(double), piece = (size_t)1 << 20;
+        const size_t np = (total + piece - 1) / piece, nbuf = std::min<size_t>(np, 4);
+        HIPCHK(c, c->h_ec.ensure(std::min(total, 4 * piece)));
+        auto issue = [&](size_t i) -> hipError_t {
+            hipError_t e = lazy_event(c->ev_ec[i % 4]);
+            if (e != hipSuccess) return e;
+            const size_t o = i * piece;
+            e = hipMemcpyAsync(c->h_ec.p + (i % 4) * piece, reinterpret_cast<const char *>(sl.d_ecorr.p) + o,
+                               std::min(piece, total - o), hipMemcpyDeviceToHost, c->stream);
+            return e == hipSuccess ? hipEventRecord(c->ev_ec[i % 4], c->stream) : e;
         };
-        for (int k = 0; k <= c->numslv; ++k) {
-            if (minuv) minuv[k] = unord(mm[2 * k]);
-            if (maxuv) maxuv[k] = unord(mm[2 * k + 1]);
+        for (size_t i = 0; i < nbuf; ++i) HIPCHK(c, issue(i));
+        for (size_t i = 0; i < np; ++i) {
+            HIPCHK(c, hipEventSynchronize(c->ev_ec[i % 4]));
+            const size_t o = i * piece;
+            std::memcpy(reinterpret_cast<char *>(ecorr) + o, c->h_ec.p + (i % 4) * piece, std::min(piece, total - o));
+            if (i + nbuf < np) HIPCHK(c, issue(i + nbuf));
         }
     }
-    if (slnuv) HIPCHK(c, hipMemcpy(slnuv, c->S().d_slnuv.p, c->numslv * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const double *r = c->h_res.p;
+    if (edens) std::memcpy(edens, r, c->ermax * sizeof(double));
+    r += c->ermax;
+    if (eself && c->esmax > 0) std::memcpy(eself, r, c->esmax * sizeof(double));
+    r += es;
+    if (scal) std::memcpy(scal, r, 4 * sizeof(double));
+    r += 4;
+    if (slnuv) std::memcpy(slnuv, r, ns * sizeof(double));
+    const unsigned int *mm = reinterpret_cast<const unsigned int *>(r + ns);
+    auto unord = [](unsigned int u) {
+        u = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
+        float f;
+        std::memcpy(&f, &u, 4);
+        return f;
+    };
+    for (int k = 0; k <= ns; ++k) {
+        if (minuv) minuv[k] = unord(mm[2 * k]);
+        if (maxuv) maxuv[k] = unord(mm[2 * k + 1]);
+    }
     return ER_OK;
 }
 
@@ -2346,7 +2466,7 @@ extern "C" int er_get_flceng(er_ctx *c, double *flceng)
     ER_NO_CAPTURE(c, "er_get_flceng");
     if (c->prm.slttype != 1 || c->S().last_nins <= 0) return fail(c, ER_E_STATE, "er_get_flceng: no soln run");
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    HIPCHK(c, hipMemcpy(flceng, c->d_flceng.p, (size_t)c->S().last_nins * c->numslv * sizeof(double), hipMemcpyDeviceToHost));
+    std::memcpy(flceng, c->h_flceng.p, (size_t)c->S().last_nins * c->numslv * sizeof(double));
     return ER_OK;
 }
 
@@ -2355,12 +2475,7 @@ extern "C" int er_clear(er_ctx *c)
     if (!c) return ER_E_ARG;
     ER_NO_CAPTURE(c, "er_clear");
     if (!c->have_mesh) return fail(c, ER_E_STATE, "er_clear: no mesh");
-    for (Slot &sl : c->slots) {
-        const int rc = slot_clear(c, sl);
-        if (rc) return rc;
-    }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return ER_OK;
+    return clear_slots(c);
 }
 
 extern "C" int er_last_error(er_ctx *c, char *code, int32_t *species, float *energy)
@@ -2633,6 +2748,13 @@ extern "C" int er_autotune(er_ctx *c, int32_t reps)
     std::memcpy(c->prof_n, n_keep, sizeof n_keep);
     c->prof = prof_keep;
     for (size_t k = 0; k < c->slots.size(); ++k) HIPCHK(c, slot_snap(c->slots[k], snap[k], c->stream, false));
+    for (size_t k = 0; k < c->slots.size(); ++k) {  // the host's view of the restored halts
+        Slot &sl = c->slots[k];
+        unsigned long long *h = c->h_halt.p + 6 * k;
+        HIPCHK(c, hipMemcpyAsync(h, sl.d_errkey.p, sizeof *h, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipMemcpyAsync(h + 1, sl.d_warnkey.p, sizeof *h, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipMemcpyAsync(h + 2, sl.d_halt.p, 4 * sizeof *h, hipMemcpyDeviceToHost, c->stream));
+    }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return rc;
 }
@@ -2910,6 +3032,10 @@ extern "C" void er_destroy(er_ctx *c)
     c->d_selfpart.release(); c->d_Ftab.release(); c->d_T.release(); c->d_phi.release();
     c->d_C.release(); c->d_w.release(); c->d_border.release(); c->d_bdesc.release(); c->d_flceng.release(); c->d_part.release(); c->d_epart.release();
     if (c->stream2) (void)hipStreamSynchronize(c->stream2);
+    for (hipEvent_t e : c->ev_up)
+        if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->ev_ec)
+        if (e) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     if (c->stream2) (void)hipStreamDestroy(c->stream2);
     if (c->ev_in) (void)hipEventDestroy(c->ev_in);

@@ -74,6 +74,7 @@ struct SlotDesc {
     unsigned int *minmax;          // minuv/maxuv as order keys
     double *edens, *ecorr, *eself, *slnuv;
     unsigned long long *errkey, *warnkey, *halt;
+    unsigned long long *hhalt;     // host memory: errkey, warnkey and halt[4] after each run
 };
 
 // the solute whose range holds x: the largest k with key(k) <= x (keys
@@ -3134,14 +3135,15 @@ __device__ __forceinline__ float weights_uv0(const WeightArgs &wa, const double 
 // engnmfc (engproc.F90:858-912); flceng; the scalar accumulators; the
 // sequential parts in n as the reference adds them (self-energy distribution,
 // slnuv); and last the halt capture.  Latency-bound (a few KB per solute):
-// one launch instead of four (5 + 17 + 5 + 4 us at 1000 insertions, WGT us
+// one launch instead of four (5 + 17 + 5 + 4 us at 1000 insertions, 17 us
 // together), with the plane partials read across the insertions.
 __global__ void __launch_bounds__(1024) k_weights(WeightArgs wa, AccRange ar, const SlotDesc *__restrict__ sd,
                                                   int ntot, const double *__restrict__ selfpart,
                                                   const float *__restrict__ selfreal,
                                                   const float *__restrict__ resself, float *u0, double *wout,
                                                   const double *__restrict__ escrd,
-                                                  const double *__restrict__ flpart, double *flceng, int NI, int nmol,
+                                                  const double *__restrict__ flpart, double *flceng,
+                                                  double *__restrict__ hflceng, int NI, int nmol,
                                                   const float *__restrict__ U)
 {
     __shared__ double r_w[16], r_t[16];
@@ -3197,7 +3199,10 @@ __global__ void __launch_bounds__(1024) k_weights(WeightArgs wa, AccRange ar, co
             double f = 0.0;
             for (int sl = lane; sl < wa.nslice; sl += 64) f += flpart[((size_t)n * wa.nslice + sl) * wa.numslv + sp];
             for (int off = 32; off > 0; off >>= 1) f += __shfl_xor(f, off, 64);
-            if (lane == 0) flceng[(size_t)n * wa.numslv + sp] = f;
+            if (lane == 0) {
+                flceng[(size_t)n * wa.numslv + sp] = f;
+                hflceng[(size_t)n * wa.numslv + sp] = f;  // host memory, for er_get_flceng
+            }
         }
     for (int off = 32; off > 0; off >>= 1) {
         sw += __shfl_xor(sw, off, 64);
@@ -3274,13 +3279,57 @@ __global__ void __launch_bounds__(1024) k_weights(WeightArgs wa, AccRange ar, co
         unsigned long long *cap = sd[k].halt;
         const unsigned long long key = __hip_atomic_load(gptr(tid == 0 ? sd[k].errkey : sd[k].warnkey),
                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (key == ~0ull || (unsigned int)(key >> 42) != (seq & 0x3fffffu) || cap[2 * tid] == key) return;
-        // the key holds the insertion within its solute
-        const int n = base + (int)((key >> 21) & 0x1fffffu), jp1 = (int)(key & 0x1fffffu);
-        const float v = jp1 == 0 ? u0[n] : U[((size_t)(n / NI) * nmol + (jp1 - 1)) * NI + (n % NI)];
-        cap[2 * tid] = key;
-        cap[2 * tid + 1] = (unsigned long long)__float_as_uint(v);
+        if (key != ~0ull && (unsigned int)(key >> 42) == (seq & 0x3fffffu) && cap[2 * tid] != key) {
+            // the key holds the insertion within its solute
+            const int n = base + (int)((key >> 21) & 0x1fffffu), jp1 = (int)(key & 0x1fffffu);
+            const float v = jp1 == 0 ? u0[n] : U[((size_t)(n / NI) * nmol + (jp1 - 1)) * NI + (n % NI)];
+            cap[2 * tid] = key;
+            cap[2 * tid + 1] = (unsigned long long)__float_as_uint(v);
+        }
+        // er_sync reads the state of the halts in host memory
+        unsigned long long *h = sd[k].hhalt;
+        h[tid] = key;
+        h[2 + 2 * tid] = cap[2 * tid];
+        h[3 + 2 * tid] = cap[2 * tid + 1];
     }
+}
+
+// er_clear: the block accumulators of up to ER_CLEAR_SLOTS solutes, one grid
+// row each
+#define ER_CLEAR_SLOTS 16
+struct ClearArgs {
+    double *edens[ER_CLEAR_SLOTS], *ecorr[ER_CLEAR_SLOTS], *eself[ER_CLEAR_SLOTS], *slnuv[ER_CLEAR_SLOTS],
+        *state[ER_CLEAR_SLOTS];
+};
+__global__ void k_clear(ClearArgs ca, int ermax, int esmax, int numslv)
+{
+    const int k = blockIdx.y;
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x, T = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = t; i < (size_t)ermax * ermax; i += T) ca.ecorr[k][i] = 0.0;
+    for (size_t i = t; i < (size_t)ermax; i += T) ca.edens[k][i] = 0.0;
+    for (size_t i = t; i < (size_t)esmax; i += T) ca.eself[k][i] = 0.0;
+    if (t < (size_t)numslv) ca.slnuv[k][t] = 0.0;
+    // engnorm, engsmpl, avslf (voffset survives, engproc.F90:336-338)
+    if (t < 3) ca.state[k][t] = 0.0;
+}
+
+// er_fetch: everything but ecorr into host memory in one launch
+// [edens | eself | state 4 | slnuv | minmax]
+__global__ void __launch_bounds__(1024) k_fetch(int ermax, int esmax, int numslv, const double *__restrict__ edens,
+                                                const double *__restrict__ eself, const double *__restrict__ state,
+                                                const double *__restrict__ slnuv,
+                                                const unsigned int *__restrict__ minmax, double *__restrict__ out)
+{
+    const int tid = threadIdx.x;
+    for (int i = tid; i < ermax; i += 1024) out[i] = edens[i];
+    out += ermax;
+    for (int i = tid; i < esmax; i += 1024) out[i] = eself[i];
+    out += esmax;
+    if (tid < 4) out[tid] = state[tid];
+    out += 4;
+    for (int i = tid; i < numslv; i += 1024) out[i] = slnuv[i];
+    unsigned int *mm = reinterpret_cast<unsigned int *>(out + numslv);
+    for (int i = tid; i < 2 * (numslv + 1); i += 1024) mm[i] = minmax[i];
 }
 
 // edens(b) += engnmfc * count (engproc.F90:943-947), sequential in n per bin
