@@ -1524,6 +1524,19 @@ template <int NI, int LPM> static hipError_t launch_gather(er_ctx *c, int n_off,
 // region must fit the 160 KB LDS (order 8: 15 x 15 x 11 points, 158 KB)
 static bool brick_order(int ord) { return ord >= 3 && ord <= 8; }
 
+// the molecules' sums of the atoms' energies that a brick gather has written
+template <int NI> static hipError_t launch_mol_reduce(er_ctx *c, int n_off, int nch)
+{
+    const bool soln = c->prm.slttype == 1;
+    const int ntile = (nch + NI - 1) / NI;
+    const int mpb = NI == 16 ? ER_MR_MPT4 * 64 : ER_MR_MPT * (256 / NI);  // molecules per block
+    hipLaunchKernelGGL((k_mol_reduce<NI>), dim3((unsigned)((c->nummol + mpb - 1) / mpb), ntile), dim3(256), 0,
+                       c->stream, c->nummol, nch, n_off, c->numatm, c->d_molbeg.p, c->d_molq.p, c->d_Eat.p,
+                       soln ? c->d_tag.p : (const int *)nullptr, (int)c->plan.desc.size(), c->d_sd.p, c->prm.screen,
+                       c->fc.volume, c->d_Ucat.p);
+    return hipGetLastError();
+}
+
 template <int ORD, int NI> static hipError_t launch_gather_brick_k(er_ctx *c, int n_off, int nch)
 {
     static_assert((size_t)(ER_BRICK + ORD - 1) * (ER_BRICK + ORD - 1) * (brick_z(ORD) + ORD - 1) * (NI / 4) * 16 <=
@@ -1545,14 +1558,27 @@ template <int ORD, int NI> static hipError_t launch_gather_brick_k(er_ctx *c, in
                        c->d_Eat.p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const bool soln = c->prm.slttype == 1;
-    const int mpb = NI == 16 ? ER_MR_MPT4 * 64 : ER_MR_MPT * (256 / NI);  // molecules per block
-    hipLaunchKernelGGL((k_mol_reduce<NI>), dim3((unsigned)((c->nummol + mpb - 1) / mpb), ntile), dim3(256),
-                       0, c->stream, c->nummol,
-                       nch, n_off, c->numatm, c->d_molbeg.p, c->d_molq.p, c->d_Eat.p,
-                       soln ? c->d_tag.p : (const int *)nullptr, (int)c->plan.desc.size(), c->d_sd.p, c->prm.screen,
-                       c->fc.volume, c->d_Ucat.p);
-    return hipGetLastError();
+    return launch_mol_reduce<NI>(c, n_off, nch);
+}
+
+// order 6: the sweeping gather (one workgroup per CU, a whole column of bricks
+// each) where the launch has four columns per CU or more.  With fewer the last
+// round of workgroups weighs too much: 6 000 atoms x 96 insertions on 40^3 (150
+// columns) took 2 % longer over all in segments of a column than in single
+// bricks, 1 600 atoms x 7 on 32^3 15.3 against 13.0 us for the gather.
+static bool sweep_pays(const er_ctx *c, int ntile)
+{
+    return (long)ntile * c->nbx * c->nby >= 4L * std::max(1, c->ncu);
+}
+
+template <int ORD, int NI> static hipError_t launch_gather_sweep_k(er_ctx *c, int n_off, int nch)
+{
+    const long total = (long)((nch + NI - 1) / NI) * c->nbx * c->nby;
+    hipLaunchKernelGGL(k_gather_sweep<ORD>, dim3((unsigned)(8 * ((total + 7) / 8))), dim3(ER_SW_NT), 0, c->stream,
+                       c->K1, c->K2, c->K3, c->nbx, c->nby, c->nbz, c->d_bstart.p, nch, c->d_brec.p, c->d_phi.p,
+                       c->numatm, c->d_Eat.p);
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : launch_mol_reduce<NI>(c, n_off, nch);
 }
 
 // order 4: the streaming gather, one workgroup per CU (its two LDS buffers
@@ -1565,14 +1591,7 @@ template <int NI> static hipError_t launch_gather_stream_k(er_ctx *c, int n_off,
                        c->d_Eat.p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const bool soln = c->prm.slttype == 1;
-    const int ntile = (nch + NI - 1) / NI;
-    const int mpb = NI == 16 ? ER_MR_MPT4 * 64 : ER_MR_MPT * (256 / NI);  // molecules per block
-    hipLaunchKernelGGL((k_mol_reduce<NI>), dim3((unsigned)((c->nummol + mpb - 1) / mpb), ntile), dim3(256), 0,
-                       c->stream, c->nummol, nch, n_off, c->numatm, c->d_molbeg.p, c->d_molq.p, c->d_Eat.p,
-                       soln ? c->d_tag.p : (const int *)nullptr, (int)c->plan.desc.size(), c->d_sd.p, c->prm.screen,
-                       c->fc.volume, c->d_Ucat.p);
-    return hipGetLastError();
+    return launch_mol_reduce<NI>(c, n_off, nch);
 }
 
 template <int NI> static hipError_t launch_hist(er_ctx *c, int n_off, int nch)
@@ -2023,7 +2042,9 @@ template <int NI> static hipError_t run_chunk(er_ctx *c, int n_off, int nch)
         case 3: return launch_gather_brick_k<3, NI>(c, n_off, nch);
         case 4: return launch_gather_stream_k<NI>(c, n_off, nch);
         case 5: return launch_gather_brick_k<5, NI>(c, n_off, nch);
-        case 6: return launch_gather_brick_k<6, NI>(c, n_off, nch);
+        case 6:
+            return sweep_pays(c, (nch + NI - 1) / NI) ? launch_gather_sweep_k<6, NI>(c, n_off, nch)
+                                                      : launch_gather_brick_k<6, NI>(c, n_off, nch);
         case 7: return launch_gather_brick_k<7, NI>(c, n_off, nch);
         case 8: return launch_gather_brick_k<8, NI>(c, n_off, nch);
         default: return launch_gather<NI, NI>(c, n_off, nch);  // 9, 10: regions beyond one wave's row

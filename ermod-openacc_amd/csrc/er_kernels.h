@@ -2219,6 +2219,223 @@ __global__ void __launch_bounds__(ER_GS_NT) k_gather_stream(int K1, int K2, int 
     }
 }
 
+// ---------------------------------------------------------------------------
+// Sweeping form of the brick gather (order 6): a workgroup owns one column of
+// bricks (8 x 8 points by x and y) and one tile, and walks it upwards in z, two
+// bricks (BZ planes) per step.  The planes lie in a ring of BZ (next step) +
+// BZ + ORD - 1 (this step) planes: while the atoms of one step are computed only
+// the BZ planes that the next one adds are on their way into the ring (43 KB),
+// where a region per brick stages BZ/2 + ORD - 1 planes (76 KB) for half the
+// atoms and waits for them.
+// The copies are issued as asm: the compiler keeps every LDS read of an array
+// behind the copies in flight into it, and here the planes read and the
+// planes written are always different ones.  Each wave waits for its own copies
+// before the barrier that ends the step.
+// Arithmetic as in k_gather_brick.  Two lanes per insertion quad share an atom
+// (even and odd x offsets): four leave a quarter of their columns empty (1526 us
+// on the first shape below).  Bound by LDS reads (66 % of the cycles busy) where
+// atoms are dense, by the staging where they are sparse: 90 000 atoms x 700
+// insertions on 72^3 1410 -> 1386 us against a region per brick, 8 100 atoms x
+// 300 insertions in a slab of a 60 x 60 x 100 grid 677 -> 424 us; one plane
+// depth less per step (BZ = 2) 1527 and 509 us, 512 threads 1455 and 438 us.
+// ---------------------------------------------------------------------------
+template <int ORD> struct Sweep {
+    static constexpr int BZ = 2 * brick_z(ORD), RS = ER_BRICK + ORD - 1, RP = 2 * BZ + ORD - 1;
+    static constexpr int NV = 4, RSU = RS * NV, PLANE = RS * RSU;  // float4 per point, row, plane
+    static constexpr int RECF = brick_rec_floats(ORD), RECU = RECF / 4, RCAP = 96;
+    static constexpr int XL = 2, NX = (ORD + XL - 1) / XL;  // lanes along the x offsets, columns per lane
+    typedef float V __attribute__((ext_vector_type(4)));
+    static_assert(RSU <= 64, "a region row is staged by one wave instruction");
+    static_assert((size_t)(RP * PLANE + 2 * RCAP * RECU) * 16 <= 160 * 1024, "ring and records fit the LDS");
+};
+#define ER_SW_NT 1024
+// one row of planes or records into LDS: lane l's 16 bytes at base + off land at
+// LDS byte address lds + 16 l
+__device__ __forceinline__ void lds_copy16(const void *base, unsigned int off, unsigned int lds)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(base)
+                 : "memory");
+}
+template <int ORD>
+__global__ void __launch_bounds__(ER_SW_NT) k_gather_sweep(int K1, int K2, int K3, int nbx, int nby, int nbz,
+                                                           const unsigned int *__restrict__ bstart, int nchunk,
+                                                           const float *__restrict__ rec,
+                                                           const float *__restrict__ phi, int natom,
+                                                           float *__restrict__ Eat)
+{
+    using S = Sweep<ORD>;
+    using VT = typename S::V;
+    constexpr int NI = 16, NT = ER_SW_NT, NW = NT / 64, APASS = NT / (S::XL * S::NV);
+    __shared__ __align__(16) float4 ring[S::RP * S::PLANE];
+    __shared__ __align__(16) float4 recs[2][S::RCAP * S::RECU];
+    // each XCD takes one contiguous eighth of the (tile, column)
+    // list, columns fastest: the columns whose planes overlap run together
+    const int ncol = nbx * nby;
+    const int total = ncol * ((nchunk + NI - 1) / NI), per = (total + 7) / 8;
+    const int v = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (v >= total) return;
+    const int col = v % ncol, tile = v / ncol;
+    const int bx = col % nbx, by = col / nbx;
+    const int ox = bx * ER_BRICK - (ORD - 1), oy = by * ER_BRICK - (ORD - 1);
+    const float4 *ph4 = reinterpret_cast<const float4 *>(phi) + (size_t)tile * K1 * K2 * K3 * S::NV;
+    const float4 *rec4 = reinterpret_cast<const float4 *>(rec);
+    VT *EatV = reinterpret_cast<VT *>(Eat);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = tid % S::NV, cx = (tid / S::NV) % S::XL, as = tid / (S::NV * S::XL);
+    const unsigned int ring_at = (unsigned int)(uintptr_t)(__attribute__((address_space(3))) void *)ring;
+    const unsigned int recs_at = (unsigned int)(uintptr_t)(__attribute__((address_space(3))) void *)&recs[0][0];
+    const int gx = wrap1(ox + lane / S::NV, K1);  // in [-RS, K1 + RS): K1 >= 16 > RS
+    const unsigned int lbyte = (unsigned int)(gx * S::NV + lane % S::NV) * 16u;
+    // plane p (counted from z = -(ORD - 1) of the whole column) lies in slot p % RP
+    auto stage_planes = [&](int p0, int n) {
+        for (int r = wv; r < n * S::RS; r += NW) {  // wave-uniform
+            const int p = p0 + r / S::RS, ry = r % S::RS;
+            const int gy = wrap1(oy + ry, K2);
+            int gz = p - (ORD - 1);
+            gz += (gz < 0) ? K3 : 0;
+            gz -= (gz >= K3) ? K3 : 0;
+            if (lane < S::RSU)
+                lds_copy16(ph4 + ((size_t)gy * K3 + gz) * K1 * S::NV, lbyte,
+                           ring_at + (unsigned int)((p % S::RP) * S::PLANE + ry * S::RSU) * 16u);
+        }
+    };
+    // a step's atoms: n of them, the first na records from a, the others from b
+    struct Atoms {
+        unsigned int a, b;
+        int na, n;
+    };
+    auto atoms_of = [&](int st) {
+        const int i = (2 * st * nby + by) * nbx + bx;
+        Atoms r;
+        r.a = bstart[i];
+        r.n = r.na = (int)(bstart[i + 1] - r.a);
+        r.b = 0;
+        if (2 * st + 1 < nbz) {
+            r.b = bstart[i + ncol];
+            r.n += (int)(bstart[i + ncol + 1] - r.b);
+        }
+        return r;
+    };
+    // the first RCAP records of a step
+    auto stage_recs = [&](const Atoms &r, int buf) {
+        const int ua = min(r.na, S::RCAP) * S::RECU, ub = min(r.n, S::RCAP) * S::RECU - ua;
+        for (int u0 = wv * 64; u0 < ua; u0 += NT)
+            if (u0 + lane < ua)
+                lds_copy16(rec4 + (size_t)r.a * S::RECU, (unsigned int)(u0 + lane) * 16u,
+                           recs_at + (unsigned int)(buf * S::RCAP * S::RECU + u0) * 16u);
+        for (int u0 = wv * 64; u0 < ub; u0 += NT)
+            if (u0 + lane < ub)
+                lds_copy16(rec4 + (size_t)r.b * S::RECU, (unsigned int)(u0 + lane) * 16u,
+                           recs_at + (unsigned int)(buf * S::RCAP * S::RECU + ua + u0) * 16u);
+    };
+    Atoms cur = atoms_of(0);
+    stage_planes(0, S::BZ + ORD - 1);
+    stage_recs(cur, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const int nst = (nbz + 1) / 2;
+    for (int st = 0; st < nst; ++st) {
+        Atoms nxt = {0, 0, 0, 0};
+        const int buf = st & 1;
+        if (st + 1 < nst) {
+            nxt = atoms_of(st + 1);
+            stage_planes((st + 1) * S::BZ + ORD - 1, S::BZ);
+            stage_recs(nxt, buf ^ 1);
+        }
+        const int pz = (st * S::BZ) % S::RP;  // slot of the lower brick's lowest plane
+        // one pass of APASS atoms from base; records from LDS or, beyond the
+        // RCAP staged ones, from global memory.  The two stay separate code: a
+        // wait for a global load would also wait for the copies in flight.
+        auto pass = [&](int base, int end, auto from_lds) __attribute__((always_inline)) {
+            const int pos = base + as;
+            const bool live = pos < end;
+            if (!__any(live)) return;
+            VT ea = VT(0.f);
+            float q = 0.f;
+            int atom = 0;
+            if (live) {
+                float f[S::RECF];
+                const size_t g = pos < cur.na ? cur.a + pos : cur.b + (pos - cur.na);
+#pragma unroll
+                for (int u = 0; u < S::RECU; ++u) {
+                    if constexpr (decltype(from_lds)::value)
+                        *reinterpret_cast<float4 *>(f + 4 * u) = recs[buf][pos * S::RECU + u];
+                    else
+                        *reinterpret_cast<float4 *>(f + 4 * u) = rec4[g * S::RECU + u];
+                }
+                q = f[3 * ORD];
+                const int li = __float_as_int(f[3 * ORD + 1]);
+                const int lx = li & 0xff, ly = (li >> 8) & 0xff, lz = (li >> 16) + (pos < cur.na ? 0 : S::BZ / 2);
+                atom = __float_as_int(f[3 * ORD + 2]);
+                int off[ORD];  // plane of stencil point c3
+                int sl = pz + lz;
+                sl -= (sl >= S::RP) ? S::RP : 0;
+#pragma unroll
+                for (int c3 = 0; c3 < ORD; ++c3) {
+                    off[c3] = sl * S::PLANE;
+                    sl = sl == 0 ? S::RP - 1 : sl - 1;
+                }
+#pragma unroll
+                for (int m = 0; m < S::NX; ++m) {
+                    // x offset c1 = cx + XL m; past the stencil w1 = 0 on a clamped column
+                    float w1 = 0.f;
+#pragma unroll
+                    for (int x = 0; x < S::XL; ++x)
+                        if (x + S::XL * m < ORD && cx == x) w1 = f[x + S::XL * m];
+                    const int c1 = min(cx + S::XL * m, ORD - 1);
+                    const VT *b0 = reinterpret_cast<const VT *>(ring) +
+                                   ((ly - (ORD - 1)) * S::RS + (lx - c1)) * S::NV + j;
+                    VT xs = VT(0.f);
+                    // the reads of the next row of points under the sums of this one
+                    VT pr2[2][ORD];
+#pragma unroll
+                    for (int c2 = 0; c2 < ORD; ++c2) pr2[0][c2] = b0[off[0] + (ORD - 1 - c2) * S::RS * S::NV];
+#pragma unroll
+                    for (int c3 = 0; c3 < ORD; ++c3) {
+                        if (c3 + 1 < ORD) {
+#pragma unroll
+                            for (int c2 = 0; c2 < ORD; ++c2)
+                                pr2[(c3 + 1) & 1][c2] = b0[off[c3 + 1] + (ORD - 1 - c2) * S::RS * S::NV];
+                        }
+                        const VT *pr = pr2[c3 & 1];
+                        VT zs = VT(0.f);
+#pragma unroll
+                        for (int c2 = 0; c2 < ORD; ++c2) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) zs[e] += f[ORD + c2] * pr[c2][e];
+                        }
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) xs[e] += f[2 * ORD + c3] * zs[e];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ea[e] += w1 * xs[e];
+                }
+            }
+            // the x-lanes of an atom, XL consecutive groups of LPP lanes; every
+            // lane of the wave takes part in the exchanges
+#pragma unroll
+            for (int off = S::XL * S::NV / 2; off >= S::NV; off >>= 1)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ea[e] += __shfl_xor(ea[e], off, 64);
+            if (live && cx == 0) {
+                VT o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = q * ea[e];
+                EatV[((size_t)tile * natom + atom) * S::NV + j] = o;
+            }
+        };
+        const int split = min(cur.n, S::RCAP);
+        for (int base = 0; base < split; base += APASS) pass(base, split, std::integral_constant<bool, true>{});
+        for (int base = split; base < cur.n; base += APASS) pass(base, cur.n, std::integral_constant<bool, false>{});
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        cur = nxt;
+    }
+}
+
 // per-molecule sum of the atom energies (atom order as in k_gather) plus the
 // residual background term (engproc.F90:979-1020); writes U
 #define ER_MR_MPT 8   // molecules per thread in k_mol_reduce
