@@ -1294,21 +1294,35 @@ template <> struct Split<96> { static constexpr int A = 8, B = 12; };
 template <> struct Split<108> { static constexpr int A = 12, B = 9; };
 template <> struct Split<128> { static constexpr int A = 8, B = 16; };
 
+// Threads of the plane kernel.  512 where three workgroups share a CU (72 x 72:
+// 601 us for 1000 insertions of five sites, 666 with 576 threads, 732 with 256;
+// 64 x 64: 226 -> 184 us for 500 against 256 threads) and, for its registers,
+// where the plane fills a CU (above 80 KB); 768 where two do (96 x 96: 1032 ->
+// 679 us for 500 against 512).  Planes below 64 x 64 keep 256 (48 x 48: 90 us,
+// 105 with 384).
+constexpr int spec2d_threads(int K2, int K3)
+{
+    const int bytes = K2 * (K3 + 1) * 8;
+    return bytes > 53 * 1024 && bytes <= 80 * 1024 ? 768 : K2 * K3 >= 4096 ? 512 : 256;
+}
+
 // the plane kernel over insertions [n_off, n_off + nch) of the run, whose T
 // rows start at insertion t_off; sparse: the scatter + forward DFT form (the
 // solutes of more than ER_SPARSE_SITES sites)
 template <int K2, int K3> static hipError_t launch_spec2d_k(er_ctx *c, int n_off, int nch, int t_off, bool sparse)
 {
     constexpr int R1 = Split<K3>::A, R2 = Split<K3>::B, C1 = Split<K2>::A, C2 = Split<K2>::B;
-    constexpr int NT = (K2 * K3 >= 5184) ? 512 : 256;  // large planes: more threads, fewer values per thread
-    const size_t lds = (size_t)K2 * (K3 + 1) * sizeof(float2) + (size_t)ER_SCH * (K2 + K3) * sizeof(float2) +
-                       (K2 + K3) * sizeof(float2) + (NT / 64) * sizeof(double);
+    constexpr int NT = spec2d_threads(K2, K3);
+    const auto bytes = [](bool sp) {
+        return (spec2d_points(K2, K3, sp) + K2 + K3) * sizeof(float2) + (NT / 64) * sizeof(double);
+    };
+    const size_t lds = bytes(sparse);
     static bool attr = false;
-    if (!attr && lds > 65536) {
+    if (!attr && bytes(true) > 65536) {
         (void)hipFuncSetAttribute((const void *)k_pme_spec2d<K2, K3, R1, R2, C1, C2, NT, false>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes(false));
         (void)hipFuncSetAttribute((const void *)k_pme_spec2d<K2, K3, R1, R2, C1, C2, NT, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes(true));
         attr = true;
     }
     const int nslot = (int)c->plan.desc.size();

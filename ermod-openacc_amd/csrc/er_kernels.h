@@ -827,6 +827,12 @@ __device__ __forceinline__ void plane_dft(float2 *plane, const float2 *t2, const
 //      of recpcal.F90:446-478, done per plane).
 //   2. FP64 half-plane self-energy partial and the engfac multiply.
 //   3. inverse DFT along axes 3 and 2; T[nl][m1][x2][x3] for stage B.
+// float2 of LDS for the plane and the sites' factors of k_pme_spec2d
+__host__ __device__ constexpr int spec2d_points(int K2, int K3, bool sparse)
+{
+    const int plane = K2 * (K3 + 1), fac = ER_SCH * (K2 + K3);
+    return sparse ? plane + fac : (plane > fac ? plane : fac);
+}
 template <int K2, int K3, int R1, int R2, int C1, int C2, int NT, bool SPARSE>
 __global__ void __launch_bounds__(NT) k_pme_spec2d(int nslot, const SlotDesc *__restrict__ sd, int ord, int K1,
                                                     int n_off,
@@ -843,9 +849,13 @@ __global__ void __launch_bounds__(NT) k_pme_spec2d(int nslot, const SlotDesc *__
     constexpr int EPT = (NE + NT - 1) / NT;
     extern __shared__ __align__(16) unsigned char smem[];
     float2 *plane = reinterpret_cast<float2 *>(smem);  // [K2][PS]
-    float2 *F2 = plane + K2 * PS;                       // [SCH][K2]: F1(m1) * F2(m2)
-    float2 *F3 = F2 + ER_SCH * K2;                      // [SCH][K3]
-    float2 *t2 = F3 + ER_SCH * K3;                      // [K2]
+    // factors [SCH][K2]: F1(m1) * F2(m2), then [SCH][K3]; in the product form
+    // they lie where the plane comes after them (80 x 80: 53 KB instead of 63,
+    // three workgroups per CU instead of two, 484 -> 409 us for 500 insertions
+    // of five sites)
+    float2 *F2 = SPARSE ? plane + K2 * PS : plane;
+    float2 *F3 = F2 + ER_SCH * K2;
+    float2 *t2 = plane + spec2d_points(K2, K3, SPARSE);  // [K2]
     float2 *t3 = t2 + K2;                               // [K3]
     double *red = reinterpret_cast<double *>(t3 + K3);  // [NT/64]
 
