@@ -1027,8 +1027,6 @@ extern "C" int er_set_solute_molecules(er_ctx *c, int32_t nslt, const int32_t *t
     return ER_OK;
 }
 
-// Morton keys of nc cells per axis: coordinates below the next power of two
-// p interleave into keys below p^3 (32^3 at most)
 // realcal_prepare's cell handling (realcal.F90:776-896) + get_inverted_cell
 static int frame_cell(er_ctx *c, const float *cell)
 {

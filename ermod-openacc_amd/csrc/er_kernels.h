@@ -1407,7 +1407,7 @@ __global__ void __launch_bounds__(ER_GEN_NT) k_pme_axis1_gen(int nchunk, int NI,
 
 // ---------------------------------------------------------------------------
 // Spatial order of the molecules (per frame): counting sort of the molecule
-// centres into NC^3 cells keyed by the Morton code of the cell, so
+// centres into NC^3 cells keyed by cell_key, so
 // that consecutive molecules are neighbours in space.  The gather walks the
 // molecules in this order (neighbouring stencils hit the same L2 lines) and
 // the pair search uses the cells as a cell list.

@@ -154,9 +154,8 @@ int er_run(er_ctx *c, int32_t mode);
  * allocating library routine: every per-run buffer of the context must
  * already hold this run's shapes (an earlier er_run of at least as many
  * insertions per solute, same launch shapes, sizes them; otherwise
- * ER_E_STATE), and the split-K partial sums of edens/ecorr and the weight
- * partials live in a 64 MiB array of the library's own that each GPU holds
- * until the process ends.  A run whose partial sums exceed it (about
+ * ER_E_STATE), and the split-K partial sums of edens/ecorr live in a 64 MiB
+ * array of the library's own that each GPU holds until the process ends.  A run whose partial sums exceed it (about
  * nslices x ermax^2 x 8 bytes with ecorr on) returns ER_E_UNSUPPORTED.
  * Results equal er_run's.  All contexts on one GPU share that array, so
  * er_run_noalloc calls that overlap on one GPU race: issue them from one
