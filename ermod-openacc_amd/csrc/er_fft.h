@@ -1,4 +1,4 @@
-// er_fft.h -- register-resident mixed-radix (2/3/4/5) Stockham FFT for one
+// er_fft.h -- register-resident mixed-radix (2/3/4/5/7) Stockham FFT for one
 // line per thread, fully unrolled at compile time so that every element and
 // every twiddle index is a constant: the line lives in VGPRs and the
 // twiddles are uniform loads from a per-length table tw[k] = exp(+2 pi i k/N)
