@@ -74,14 +74,19 @@ template <typename T> struct HBuf {
     HBuf(const HBuf &) = delete;
     HBuf &operator=(const HBuf &) = delete;
     ~HBuf() { release(); }
-    hipError_t ensure(size_t count)
+    // room for count elements, the first `keep` as they were; the old buffer
+    // stays if the new one cannot be had
+    hipError_t ensure(size_t count, size_t keep = 0)
     {
         if (count <= n && p) return hipSuccess;
+        T *q = nullptr;
+        const hipError_t e = hipHostMalloc((void **)&q, std::max<size_t>(count, 1) * sizeof(T), hipHostMallocDefault);
+        if (e != hipSuccess) return e;
+        if (keep) std::memcpy(q, p, keep * sizeof(T));
         release();
-        const hipError_t e = hipHostMalloc((void **)&p, std::max<size_t>(count, 1) * sizeof(T), hipHostMallocDefault);
-        if (e == hipSuccess) n = count;
-        else p = nullptr;
-        return e;
+        p = q;
+        n = count;
+        return hipSuccess;
     }
     void release()
     {
@@ -1022,7 +1027,8 @@ extern "C" int er_set_solute_molecules(er_ctx *c, int32_t nslt, const int32_t *t
     c->S().nslt = ns;
     HIPCHK(c, hipStreamSynchronize(c->stream));  // a run in flight may still read the list
     HIPCHK(c, c->d_tag.ensure(nslt));
-    HIPCHK(c, c->h_flceng.ensure((size_t)nslt * c->numslv));
+    // er_get_flceng goes on giving the last run's values
+    HIPCHK(c, c->h_flceng.ensure((size_t)nslt * c->numslv, (size_t)std::max(0, c->S().last_nins) * c->numslv));
     HIPCHK(c, hipMemcpy(c->d_tag.p, c->tagslt.data(), nslt * sizeof(int), hipMemcpyHostToDevice));
     return ER_OK;
 }
