@@ -569,13 +569,12 @@ static int slot_state_init(er_ctx *c, Slot &sl)
     return ER_OK;
 }
 
-// the host's view of the halts: none (no run is in flight)
-static hipError_t halt_mirror_init(er_ctx *c)
+// the host's view of the halts, for nslot slots: none (no run is in flight)
+static hipError_t halt_mirror_init(er_ctx *c, size_t nslot)
 {
-    const size_t n = 6 * c->slots.size();
-    const hipError_t e = c->h_halt.ensure(n);
+    const hipError_t e = c->h_halt.ensure(6 * nslot);
     if (e != hipSuccess) return e;
-    for (size_t k = 0; k < n; ++k) c->h_halt.p[k] = ~0ull;
+    for (size_t k = 0; k < 6 * nslot; ++k) c->h_halt.p[k] = ~0ull;
     return hipSuccess;
 }
 
@@ -821,7 +820,7 @@ extern "C" int er_create(const er_topology *topo, const er_params *prm, er_ctx *
     {
         const int rc = slot_state_init(c, c->slots[0]);
         if (rc) return bad(rc);
-        HIPCHK(c, halt_mirror_init(c));
+        HIPCHK(c, halt_mirror_init(c, 1));
     }
     // Accumulator layout of the FP64 MFMA: each output register of a known
     // product names its own (row, col); use the MFMA path only if the
@@ -938,14 +937,22 @@ extern "C" int er_set_mesh(er_ctx *c, const int32_t *uvmax, const int32_t *uvsof
     return er_clear(c);
 }
 
-static int set_slot_solute(er_ctx *c, Slot &sl, int32_t nsite, const int32_t *ljtype, const float *charge)
+static int check_solute(er_ctx *c, int32_t nsite, const int32_t *ljtype, const float *charge)
 {
     if (nsite <= 0 || !ljtype || !charge) return fail(c, ER_E_ARG, "er_set_solute: bad arguments");
+    for (int s = 0; s < nsite; ++s)
+        if (ljtype[s] < 1 || ljtype[s] > c->ntype) return fail(c, ER_E_ARG, "er_set_solute: ljtype out of range");
+    return ER_OK;
+}
+
+static int set_slot_solute(er_ctx *c, Slot &sl, int32_t nsite, const int32_t *ljtype, const float *charge)
+{
+    const int rc = check_solute(c, nsite, ljtype, charge);
+    if (rc) return rc;
     std::vector<int> lj(nsite);
     float q = 0.f;
     for (int s = 0; s < nsite; ++s) {
         lj[s] = ljtype[s] - 1;
-        if (lj[s] < 0 || lj[s] >= c->ntype) return fail(c, ER_E_ARG, "er_set_solute: ljtype out of range");
         q += charge[s];
     }
     sl.qslt = q;
@@ -976,21 +983,35 @@ extern "C" int er_set_solutes(er_ctx *c, int32_t nsolute, const int32_t *nsite, 
     ++c->alloc_gen;
     if (c->prm.slttype == 1) return fail(c, ER_E_STATE, "er_set_solutes: only for refs runs");
     if (nsolute <= 0 || !nsite || !ljtype || !charge) return fail(c, ER_E_ARG, "er_set_solutes: bad arguments");
+    // a refused call changes nothing: every solute is looked at first
+    size_t off = 0;
+    for (int k = 0; k < nsolute; ++k) {
+        const int rc = check_solute(c, nsite[k], ljtype + off, charge + off);
+        if (rc) return rc;
+        off += (size_t)nsite[k];
+    }
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    // er_sync and the runs address the mirror by slot: it covers them before they exist
+    HIPCHK(c, halt_mirror_init(c, std::max((size_t)nsolute, c->slots.size())));
     for (size_t k = (size_t)nsolute; k < c->slots.size(); ++k) c->slots[k].release();
     c->slots.resize(nsolute);
     c->cur = 0;
-    size_t off = 0;
+    off = 0;
     for (int k = 0; k < nsolute; ++k) {
         Slot &sl = c->slots[k];
+        sl.have_ins = false;
         int rc = set_slot_solute(c, sl, nsite[k], ljtype + off, charge + off);
         if (!rc) rc = slot_state_init(c, sl);
         if (!rc && c->have_mesh) rc = slot_acc_alloc(c, sl);
-        if (rc) return rc;
-        sl.have_ins = false;
+        if (rc) {  // out of memory: the slots that are whole stay, slot 1 (er_create's) without a solute at the least
+            for (size_t j = std::max(1, k); j < c->slots.size(); ++j) c->slots[j].release();
+            c->slots.resize(std::max(1, k));
+            for (Slot &s : c->slots) s.have_ins = false;
+            if (k == 0) c->slots[0].nslt = 0;
+            return rc;
+        }
         off += (size_t)nsite[k];
     }
-    HIPCHK(c, halt_mirror_init(c));
     const int rc = c->have_mesh ? clear_slots(c) : ER_OK;
     if (rc) return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream));

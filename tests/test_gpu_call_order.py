@@ -1,4 +1,5 @@
-"""Calls between runs: what er_get_flceng gives after the solute list grows."""
+"""Calls between runs: what er_get_flceng gives after the solute list grows, and
+a context after a call that it refused."""
 import numpy as np
 import pytest
 
@@ -24,3 +25,46 @@ def test_flceng_outlives_a_longer_solute_list():
     ctx.run(capi.ER_BATCHED)
     np.testing.assert_allclose(ctx.flceng(900)[:2], before, rtol=1e-6)
     ctx.close()
+
+
+def _refs_ctx(w, solutes):
+    ctx = capi.Context(w.topo, U.workload_params(w))
+    ctx.set_mesh(*w.uvmax_uvsoft_uvcrd())
+    ctx.set_solutes(solutes)
+    return ctx
+
+
+def _run(ctx, w, nsolute, nins=5):
+    ctx.set_frame(w.frame(0), w.cell)
+    for k in range(nsolute):
+        ctx.select_solute(k)
+        ctx.set_insertions(w.insertions(0)[k:k + nins])
+    ctx.run(capi.ER_BATCHED)
+    ctx.sync()
+    out = []
+    for k in range(nsolute):
+        ctx.select_solute(k)
+        out.append((ctx.uvengy(), ctx.fetch()))
+    return out
+
+
+@pytest.mark.parametrize("before,refused", [(1, 2), (1, 40), (3, 2)])
+def test_refused_solutes_change_nothing(before, refused):
+    """er_set_solutes with a bad last solute: no halt out of nowhere, and the
+    context runs, clears and fetches as if the call had not been made."""
+    w = synth.refs_water(0, 1000, 31.04, 8, 1, 32)
+    good = (w.topo.slt_ljtype, w.topo.slt_charge32)
+    bad = (np.full(5, w.topo.ntype), w.topo.slt_charge32)  # 0-based: one past the types
+    want = _refs_ctx(w, [good] * before)
+    ctx = _refs_ctx(w, [good] * before)
+    with pytest.raises(capi.ErError) as ei:
+        ctx.set_solutes([good] * (refused - 1) + [bad])
+    assert ei.value.status == capi.ER_E_ARG
+    ctx.sync()
+    ctx.clear()
+    for (ua, ga), (ub, gb) in zip(_run(ctx, w, before), _run(want, w, before), strict=True):
+        np.testing.assert_array_equal(ua[0], ub[0])
+        np.testing.assert_array_equal(ga["edens"], gb["edens"])
+        assert ga["engnorm"] == gb["engnorm"]
+    ctx.close()
+    want.close()
