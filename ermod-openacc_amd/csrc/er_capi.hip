@@ -864,26 +864,26 @@ extern "C" int er_set_mesh(er_ctx *c, const int32_t *uvmax, const int32_t *uvsof
     ER_NO_CAPTURE(c, "er_set_mesh");
     ++c->alloc_gen;
     if (!uvmax || !uvsoft || !uvcrd) return fail(c, ER_E_ARG, "er_set_mesh: null argument");
+    // a refused mesh changes nothing: the accumulators have the old one's sizes
+    int tot = 0;
+    for (int k = 0; k < c->numslv; ++k) {
+        if (uvmax[k] <= 0) return fail(c, ER_E_ARG, "er_set_mesh: uvmax must be positive");
+        if (uvmax[k] > 65535) return fail(c, ER_E_ARG, "er_set_mesh: more than 65535 bins for species %d", k + 1);
+        for (int b = 1; b < uvmax[k]; ++b)
+            if (!(uvcrd[tot + b - 1] < uvcrd[tot + b]))
+                return fail(c, ER_E_ARG, "er_set_mesh: mesh of species %d not strictly increasing", k + 1);
+        tot += uvmax[k];
+    }
+    if (c->prm.selfcal == 1 && (!escrd || esmax <= 0)) return fail(c, ER_E_ARG, "er_set_mesh: selfcal needs escrd");
+    c->have_mesh = false;  // until every buffer has the new sizes
     c->uvmax.assign(uvmax, uvmax + c->numslv);
     c->uvsoft.assign(uvsoft, uvsoft + c->numslv);
     c->idmin.assign(c->numslv, 0);
-    int tot = 0;
-    for (int k = 0; k < c->numslv; ++k) {
-        if (c->uvmax[k] <= 0) return fail(c, ER_E_ARG, "er_set_mesh: uvmax must be positive");
-        c->idmin[k] = tot;
-        tot += c->uvmax[k];
-    }
+    for (int k = 1; k < c->numslv; ++k) c->idmin[k] = c->idmin[k - 1] + c->uvmax[k - 1];
     c->ermax = tot;
     c->uvcrd.assign(uvcrd, uvcrd + tot);
-    for (int k = 0; k < c->numslv; ++k)
-        for (int b = 1; b < c->uvmax[k]; ++b)
-            if (!(c->uvcrd[c->idmin[k] + b - 1] < c->uvcrd[c->idmin[k] + b]))
-                return fail(c, ER_E_ARG, "er_set_mesh: mesh of species %d not strictly increasing", k + 1);
     c->esmax = (c->prm.selfcal == 1) ? esmax : 0;
-    if (c->prm.selfcal == 1) {
-        if (!escrd || esmax <= 0) return fail(c, ER_E_ARG, "er_set_mesh: selfcal needs escrd");
-        c->escrd.assign(escrd, escrd + esmax);
-    }
+    if (c->prm.selfcal == 1) c->escrd.assign(escrd, escrd + esmax);
     hipStream_t s = c->stream;
     HIPCHK(c, c->d_uvcrd.ensure(tot));
     HIPCHK(c, hipMemcpyAsync(c->d_uvcrd.p, c->uvcrd.data(), tot * sizeof(double), hipMemcpyHostToDevice, s));
@@ -900,7 +900,6 @@ extern "C" int er_set_mesh(er_ctx *c, const int32_t *uvmax, const int32_t *uvsof
         // bin brackets: bucket b holds the floats whose order key has top bits b
         std::vector<unsigned short> lut((size_t)c->numslv * ER_LUT_N);
         for (int k = 0; k < c->numslv; ++k) {
-            if (c->uvmax[k] > 65535) return fail(c, ER_E_ARG, "er_set_mesh: more than 65535 bins for species %d", k + 1);
             const float *m0 = mf.data() + c->idmin[k], *m1 = m0 + c->uvmax[k];
             for (int b = 0; b < ER_LUT_N - 1; ++b) {
                 const uint32_t key = (uint32_t)b << (32 - ER_LUT_BITS);  // smallest order key of the bucket
@@ -925,7 +924,6 @@ extern "C" int er_set_mesh(er_ctx *c, const int32_t *uvmax, const int32_t *uvsof
     HIPCHK(c, c->d_escrd.ensure(std::max(1, c->esmax)));
     if (c->esmax > 0)
         HIPCHK(c, hipMemcpyAsync(c->d_escrd.p, c->escrd.data(), c->esmax * sizeof(double), hipMemcpyHostToDevice, s));
-    c->ermax = tot;
     for (Slot &sl : c->slots) {
         const int rc = slot_acc_alloc(c, sl);
         if (rc) return rc;

@@ -230,13 +230,13 @@ class Context:
             raise ErError(rc, self.L.er_error_string(self.h).decode(), code.value.decode())
 
     def set_mesh(self, uvmax, uvsoft, uvcrd, escrd=None):
-        self._mesh = (np.ascontiguousarray(uvmax, np.int32), np.ascontiguousarray(uvsoft, np.int32),
-                      np.ascontiguousarray(uvcrd, np.float64),
-                      None if escrd is None else np.ascontiguousarray(escrd, np.float64))
-        um, us, uc, es = self._mesh
-        self.ermax = int(um.sum())
-        self.esmax = 0 if es is None else int(es.size)
-        self._check(self.L.er_set_mesh(self.h, _ptr(um), _ptr(us), _ptr(uc), self.esmax, _ptr(es)))
+        mesh = (np.ascontiguousarray(uvmax, np.int32), np.ascontiguousarray(uvsoft, np.int32),
+                np.ascontiguousarray(uvcrd, np.float64),
+                None if escrd is None else np.ascontiguousarray(escrd, np.float64))
+        um, us, uc, es = mesh
+        esmax = 0 if es is None else int(es.size)
+        self._check(self.L.er_set_mesh(self.h, _ptr(um), _ptr(us), _ptr(uc), esmax, _ptr(es)))
+        self._mesh, self.ermax, self.esmax = mesh, int(um.sum()), esmax
 
     def set_solute(self, ljtype0, charge32):
         lj = np.ascontiguousarray(np.asarray(ljtype0) + 1, np.int32)

@@ -68,3 +68,24 @@ def test_refused_solutes_change_nothing(before, refused):
         assert ga["engnorm"] == gb["engnorm"]
     ctx.close()
     want.close()
+
+
+def test_refused_mesh_changes_nothing():
+    """er_set_mesh with a longer mesh that does not increase: the context
+    clears, runs and fetches with the mesh it had."""
+    w = synth.refs_water(0, 1000, 31.04, 8, 1, 32)
+    good = (w.topo.slt_ljtype, w.topo.slt_charge32)
+    want, ctx = _refs_ctx(w, [good]), _refs_ctx(w, [good])
+    uvmax, uvsoft, uvcrd = w.uvmax_uvsoft_uvcrd()
+    crd = np.concatenate([uvcrd, uvcrd[-1] + np.arange(1.0, 4000.0), [uvcrd[-1]]])
+    with pytest.raises(capi.ErError) as ei:
+        ctx.set_mesh(np.array([crd.size], np.int32), uvsoft, crd)
+    assert ei.value.status == capi.ER_E_ARG
+    ctx.clear()
+    (ua, ga), = _run(ctx, w, 1)
+    (ub, gb), = _run(want, w, 1)
+    np.testing.assert_array_equal(ua[0], ub[0])
+    for key in ("edens", "ecorr"):
+        np.testing.assert_array_equal(ga[key], gb[key])
+    ctx.close()
+    want.close()
