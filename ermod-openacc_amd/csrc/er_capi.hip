@@ -875,6 +875,7 @@ extern "C" int er_set_mesh(er_ctx *c, const int32_t *uvmax, const int32_t *uvsof
         tot += uvmax[k];
     }
     if (c->prm.selfcal == 1 && (!escrd || esmax <= 0)) return fail(c, ER_E_ARG, "er_set_mesh: selfcal needs escrd");
+    HIPCHK(c, hipStreamSynchronize(c->stream));  // a run in flight bins with the old one
     c->have_mesh = false;  // until every buffer has the new sizes
     c->uvmax.assign(uvmax, uvmax + c->numslv);
     c->uvsoft.assign(uvsoft, uvsoft + c->numslv);

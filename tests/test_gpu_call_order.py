@@ -89,3 +89,21 @@ def test_refused_mesh_changes_nothing():
         np.testing.assert_array_equal(ga[key], gb[key])
     ctx.close()
     want.close()
+
+
+def test_mesh_waits_for_the_run():
+    """er_set_mesh after a run and a clear, neither of which waits: the run
+    bins with the mesh it began with, so the new one, which starts above every
+    energy, halts nothing."""
+    w = synth.refs_water(0, 1000, 31.04, 2000, 1, 32)
+    ctx = _refs_ctx(w, [(w.topo.slt_ljtype, w.topo.slt_charge32)])
+    ctx.set_frame(w.frame(0), w.cell)
+    ctx.set_insertions(w.insertions(0))
+    ctx.run(capi.ER_BATCHED)
+    ctx.sync()
+    uvmax, uvsoft, uvcrd = w.uvmax_uvsoft_uvcrd()
+    ctx.run(capi.ER_BATCHED)
+    ctx.clear()
+    ctx.set_mesh(uvmax, uvsoft, 1.0e30 + 1.0e28 * np.arange(uvcrd.size))
+    ctx.sync()
+    ctx.close()
