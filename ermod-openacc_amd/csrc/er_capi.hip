@@ -2218,6 +2218,30 @@ static hipError_t run_accumulate(er_ctx *c, AccRange ar)
     return hipGetLastError();
 }
 
+// Where a run's insertion coordinates lie: in the context's own buffer or in
+// memory of this device, which the kernels read in place; anywhere else (host
+// memory, another device's), which only a copy reads; or in an allocation that
+// ends before them.
+enum class InsAt { HERE, ELSEWHERE, SHORT };
+static InsAt insertions_at(const Slot &sl, size_t bytes)
+{
+    const float *p = sl.d_sltpos;
+    if (p == sl.d_sltpos_own.p && bytes <= sl.d_sltpos_own.n * sizeof(float)) return InsAt::HERE;
+    hipPointerAttribute_t at{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || hipPointerGetAttributes(&at, p) != hipSuccess ||
+        at.type != hipMemoryTypeDevice || at.device != dev ||
+        hipMemGetAddressRange(&base, &size, const_cast<float *>(p)) != hipSuccess) {
+        (void)hipGetLastError();
+        return InsAt::ELSEWHERE;
+    }
+    const size_t off = (size_t)(reinterpret_cast<const char *>(p) - static_cast<const char *>(base));
+    if (off + bytes > size) return InsAt::SHORT;
+    return reinterpret_cast<uintptr_t>(p) % alignof(float) ? InsAt::ELSEWHERE : InsAt::HERE;
+}
+
 // one run over the solutes `todo` of the frame: per-insertion preparation,
 // the reciprocal part in chunks, pairs, histograms and accumulation, each a
 // single launch over every solute (the plain path: one insertion at a time)
@@ -2239,6 +2263,17 @@ static int run_slots(er_ctx *c, const std::vector<int> &todo, int mode)
     if ((rc = ensure_run_buffers(c, chunk))) return rc;
     if ((rc = upload_plan(c))) return rc;
     const SlotDesc *sd = c->d_sd.p;
+    // the insertions' coordinates: in place, or copied end to end
+    bool copied = nslot > ER_INS_PTRS;
+    if (!soln)
+        for (int i = 0; i < nslot; ++i) {
+            const Slot &sl = c->slots[P.order[i]];
+            const InsAt at = insertions_at(sl, (size_t)P.desc[i].nins * sl.nslt * 3 * sizeof(float));
+            if (at == InsAt::SHORT)
+                return fail(c, ER_E_HIP, "er_run: the device memory of solute %d's insertions ends before them",
+                            P.order[i] + 1);
+            copied = copied || at == InsAt::ELSEWHERE;
+        }
     {
         ProfScope ps(c, ER_K_PREP);
         HIPCHK(c, prep_frame(c));
@@ -2246,7 +2281,7 @@ static int run_slots(er_ctx *c, const std::vector<int> &todo, int mode)
         InsSource src{};
         int maxslt = 0;
         if (!soln) {
-            if (nslot > ER_INS_PTRS) src.cat = c->d_sltcat.p;  // the insertions' coordinates, solutes end to end
+            if (copied) src.cat = c->d_sltcat.p;
             for (int i = 0; i < nslot; ++i) {
                 const Slot &sl = c->slots[P.order[i]];
                 if (src.cat)

@@ -363,7 +363,8 @@ __global__ void __launch_bounds__(256) k_prep_frame(int natom, int nab, const fl
 }
 
 // The solutes' insertion coordinates of a run, by slot; beyond ER_INS_PTRS
-// slots they are copied end to end first (cat).
+// slots, or where this device cannot read them in place, they are copied end
+// to end first (cat).
 #define ER_INS_PTRS 16
 struct InsSource {
     const float *slot[ER_INS_PTRS];

@@ -1,7 +1,11 @@
-"""Calls between runs: what er_get_flceng gives after the solute list grows, and
-a context after a call that it refused."""
+"""Calls between runs: what er_get_flceng gives after the solute list grows,
+a context after a call that it refused, inputs where the kernels cannot reach
+them."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
 import erutil as U
 from erdst_gpu import capi, synth
@@ -106,4 +110,38 @@ def test_mesh_waits_for_the_run():
     ctx.clear()
     ctx.set_mesh(uvmax, uvsoft, 1.0e30 + 1.0e28 * np.arange(uvcrd.size))
     ctx.sync()
+    ctx.close()
+
+
+def test_insertions_device_memory_ends_before_them():
+    """er_set_insertions_device on an allocation of fewer insertions than it
+    names: er_run refuses, as the copy that it once made did, and goes on with
+    the right number; a pointer to page-locked host memory is copied."""
+    w = synth.refs_water(0, 1000, 31.04, 40, 1, 32)
+    good = (w.topo.slt_ljtype, w.topo.slt_charge32)
+    ctx = _refs_ctx(w, [good])
+    x = np.ascontiguousarray(w.insertions(0), np.float32)
+    ctx.set_frame(w.frame(0), w.cell)
+    ctx.set_insertions(x)
+    ctx.run(capi.ER_BATCHED)
+    want = ctx.uvengy()[0]
+    hip = capi.load()  # finds the HIP runtime that it links
+    dev = ctypes.c_void_p()
+    assert hip.hipMalloc(ctypes.byref(dev), ctypes.c_size_t(x[:10].nbytes)) == 0
+    try:
+        assert hip.hipMemcpy(dev, ctypes.c_void_p(x.ctypes.data), ctypes.c_size_t(x[:10].nbytes), 1) == 0
+        for mode in (capi.ER_BATCHED, capi.ER_PLAIN):
+            ctx.set_insertions_device(11, dev.value)
+            with pytest.raises(capi.ErError) as ei:
+                ctx.run(mode)
+            assert ei.value.status == capi.ER_E_HIP
+        ctx.set_insertions_device(10, dev.value)
+        ctx.run(capi.ER_BATCHED)
+        np.testing.assert_array_equal(ctx.uvengy()[0], want[:10])
+    finally:
+        hip.hipFree(dev)
+    pinned = torch.from_numpy(x).pin_memory()
+    ctx.set_insertions_device(40, pinned.data_ptr())
+    ctx.run(capi.ER_BATCHED)
+    np.testing.assert_array_equal(ctx.uvengy()[0], want)
     ctx.close()
