@@ -2777,17 +2777,25 @@ __device__ __forceinline__ float molecule_pair_sum_lds(const PairArgs &pa, const
     return e;
 }
 
+// Where a thread's search stands: its cell, and how many of the cell's
+// molecules it has dealt with.
+struct PairScan {
+    int c, p;
+};
+
 // Pair search, first half (both kernels): the candidate molecules of one
-// (insertion, part) block, handed to take(j, m) one by one with their bounding
-// spheres.  Part p of nsplit scans the cells c with c % nsplit == p.
+// (insertion, part) block, handed to take(j) one by one.  Part p of nsplit
+// scans the cells c with c % nsplit == p, thread t from at = {p + t nsplit, 0}.  A
+// take that returns false ends the thread's search at that molecule, where a
+// further call with the same `at` begins.
 template <class TAKE>
 __device__ __forceinline__ void pair_candidates(const PairArgs &pa, const FrameConst &fc, const float4 &ref,
-                                                float cut, int part, int skipmol, float rmolmax,
+                                                float cut, PairScan &at, int skipmol, float rmolmax,
                                                 const unsigned int *__restrict__ cstart,
                                                 const int *__restrict__ perm, const float4 *__restrict__ molref,
                                                 TAKE take)
 {
-    const int tid = threadIdx.x, NT = blockDim.x;
+    const int NT = blockDim.x;
     int cx, cy, cz;
     site_cell(fc, ref.x, ref.y, ref.z, pa.nc, cx, cy, cz);
     // a molecule centre within distance d of the search centre lies at most
@@ -2796,7 +2804,8 @@ __device__ __forceinline__ void pair_candidates(const PairArgs &pa, const FrameC
     const int span = min(2 * nreach + 1, pa.nc);  // distinct cells per axis
     const int lo = (span == pa.nc) ? 0 : -nreach;
     const int ncell = span * span * span;
-    for (int c = part + tid * pa.nsplit; c < ncell; c += NT * pa.nsplit) {
+    for (; at.c < ncell; at.c += NT * pa.nsplit, at.p = 0) {
+        const int c = at.c;
         const int dx = c % span, dy = (c / span) % span, dz = c / (span * span);
         // cx + lo + dx lies in [-nreach, nc + nreach) with nreach < nc (or lo = 0):
         // one conditional wrap
@@ -2804,7 +2813,7 @@ __device__ __forceinline__ void pair_candidates(const PairArgs &pa, const FrameC
         const unsigned int key = cell_key(qx, qy, qz, pa.nc);
         const unsigned int p0 = cstart[key], p1 = cstart[key + 1];
         // the cell's molecules four at a time: indices, then centres
-        for (unsigned int pb = p0; pb < p1; pb += 4) {
+        for (unsigned int pb = p0 + at.p; pb < p1; pb += 4) {
             int jk[4];
             float4 mk[4];
 #pragma unroll
@@ -2819,7 +2828,10 @@ __device__ __forceinline__ void pair_candidates(const PairArgs &pa, const FrameC
                 float ddx = m.x - ref.x, ddy = m.y - ref.y, ddz = m.z - ref.z;
                 min_image(fc, ddx, ddy, ddz);
                 const float lim = cut + m.w;
-                if (ddx * ddx + ddy * ddy + ddz * ddz <= lim * lim) take(j);
+                if (ddx * ddx + ddy * ddy + ddz * ddz <= lim * lim && !take(j)) {
+                    at.p = (int)(pb + k - p0);
+                    return;
+                }
             }
         }
     }
@@ -2883,11 +2895,13 @@ __global__ void __launch_bounds__(256) k_pairs(PairArgs pa0, int blk0, int nslot
                       : molecule_pair_sum(pa, fc, 0, j, molbeg, posu, ljtype, insposu, sltlj, slt_a0, soln, ljene,
                                           ljlensq);
     };
-    pair_candidates(pa, fc, ref, cut, part, skipmol, rmolmax[0], cstart, perm, molref, [&](int j) __attribute__((always_inline)) {
+    PairScan at{part + tid * pa.nsplit, 0};
+    pair_candidates(pa, fc, ref, cut, at, skipmol, rmolmax[0], cstart, perm, molref, [&](int j) __attribute__((always_inline)) {
         const int slot = atomicAdd(&ncand, 1);
         if (slot < ER_PAIR_CAP) cand[slot] = j;
         else  // list full: evaluate in place (same arithmetic, same single owner)
             U[urow + (size_t)j * pa.NI] += pair_sum(j);
+        return true;
     });
     __syncthreads();
     const int nc = min(ncand, ER_PAIR_CAP);
@@ -2975,14 +2989,12 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
     __syncthreads();
     const int nclu = (pa.nslt + 7) >> 3;
     if (in_lds && tid < nclu) clu[tid] = site_sphere(fc, [&](int a) { return sx[a]; }, tid * 8, min(tid * 8 + 8, pa.nslt), 0, 1);
-    pair_candidates(pa, fc, ref, cut, part, skipmol, rmolmax[0], cstart, perm, molref, [&](int j) __attribute__((always_inline)) {
-        if (atomicAdd(&ncand, 1) < ER_PAIR_CAP) {
-            if (molbeg[j + 1] - molbeg[j] <= ER_PM_ATOMS) cand[atomicAdd(&nsmall, 1)] = j;
-            else cand[ER_PAIR_CAP - 1 - atomicAdd(&nlarge, 1)] = j;
-        } else {  // list full: evaluate in place, same single owner
-            U[urow + (size_t)j * pa.NI] += molecule_pair_sum(pa, fc, 0, j, molbeg, posu, ljtype, insposu, sltlj,
-                                                              slt_a0, soln, ljene, ljlensq);
-        }
+    PairScan at{part + tid * pa.nsplit, 0};
+    pair_candidates(pa, fc, ref, cut, at, skipmol, rmolmax[0], cstart, perm, molref, [&](int j) __attribute__((always_inline)) {
+        if (atomicAdd(&ncand, 1) >= ER_PAIR_CAP) return false;  // list full
+        if (molbeg[j + 1] - molbeg[j] <= ER_PM_ATOMS) cand[atomicAdd(&nsmall, 1)] = j;
+        else cand[ER_PAIR_CAP - 1 - atomicAdd(&nlarge, 1)] = j;
+        return true;
     });
     __syncthreads();
     const int ns = nsmall, nlg = nlarge;
@@ -3128,6 +3140,46 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
                 for (int off = GS / 2; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
                 if (gl == 0 && c0 + w0 + grp < ns) U[urow + (size_t)cand[c0 + w0 + grp] * pa.NI] += e;
             }
+        }
+    }
+    // More candidates than the list holds: the search goes on where it stopped,
+    // one list after the other, a wave per molecule.  Lane g adds its sites g,
+    // g + 64, ... and the tree is that of 64 lanes, which is the orders above
+    // (lanes without a site add +0 to it), so it is chance that decides which
+    // molecules come here and not their sums.  Rounds of the code above would
+    // be the faster form, but around it the compiler keeps the loop's
+    // constants in 26 more registers, a workgroup less per CU for every launch.
+    while (ncand > ER_PAIR_CAP) {  // uniform: no one adds to it between barriers
+        __syncthreads();
+        if (tid == 0) ncand = 0;
+        __syncthreads();
+        pair_candidates(pa, fc, ref, cut, at, skipmol, rmolmax[0], cstart, perm, molref, [&](int j) __attribute__((always_inline)) {
+            const int slot = atomicAdd(&ncand, 1);
+            if (slot >= ER_PAIR_CAP) return false;
+            cand[slot] = j;
+            return true;
+        });
+        __syncthreads();
+        for (int c = wv; c < min(ncand, ER_PAIR_CAP); c += NT >> 6) {
+            const int jm = __builtin_amdgcn_readfirstlane(cand[c]);
+            const int b1 = molbeg[jm + 1];
+            float e = 0.0f;
+            for (int st = lane; st < pa.nslt; st += 64) {
+                const uint4 xu = site_u(st);
+                const int ti = site_t(st);
+                float es = 0.0f;
+                for (int bb = molbeg[jm]; bb < b1; ++bb) {
+                    const uint4 xb = posu[bb];
+                    const int tj = ljtype[bb];
+                    const float d2 = lattice_d2(fc, xu, xb);
+                    if (!(d2 > skip2))
+                        es += pair_energy(pa.pp, d2, __uint_as_float(xu.w), __uint_as_float(xb.w),
+                                          ljene[ti + pa.ntype * tj], ljlensq[ti + pa.ntype * tj]);
+                }
+                e += es;
+            }
+            for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
+            if (lane == 0) U[urow + (size_t)jm * pa.NI] += e;
         }
     }
 }
