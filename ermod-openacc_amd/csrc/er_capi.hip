@@ -1861,10 +1861,10 @@ static void ecorr_slices(const er_ctx *c, int nch, int &kper, int &nks)
 static int pair_split(const er_ctx *c, const Slot &sl, int nins, bool batched)
 {
     if (batched && sl.pair_split > 0) return sl.pair_split;
-    auto fill = [&](int blocks) { return (blocks + nins - 1) / nins; };
-    if (sl.nslt > 64) return std::max(8, std::min({256, fill(32 * 256), std::max(16, c->nummol / 32)}));
-    if (sl.nslt > 8) return std::max(4, std::min({256, fill(8 * 256), std::max(16, c->nummol / 32)}));
-    return std::max(1, std::min({64, fill(4 * 256), std::max(16, c->nummol / 128)}));
+    auto fill = [&](int per_cu) { return (per_cu * std::max(1, c->ncu) + nins - 1) / nins; };
+    if (sl.nslt > 64) return std::max(8, std::min({256, fill(32), std::max(16, c->nummol / 32)}));
+    if (sl.nslt > 8) return std::max(4, std::min({256, fill(8), std::max(16, c->nummol / 32)}));
+    return std::max(1, std::min({64, fill(4), std::max(16, c->nummol / 128)}));
 }
 
 // The run's solutes end to end: the solutes of few sites first (dense plane
