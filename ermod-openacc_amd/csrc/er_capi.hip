@@ -1487,10 +1487,11 @@ template <int NI> static hipError_t launch_axis1(er_ctx *c, int nch)
 {
     if (!fft_len_ok(c->K1) && NI == 16 && c->lp[0].nf) {
         // the factored kernel: the most lines per workgroup (64-byte runs of T
-        // at eight) whose LDS still leaves three workgroups per CU.  60 x 60 x
+        // at eight) whose LDS still leaves three workgroups per CU, at least
+        // the two that share a transform (71 KB at K1 = 512).  60 x 60 x
         // 100, 300 insertions: 258 us (3.4 TB/s over T and phi) against 681 us direct.
         int rsh = 3;
-        while (rsh > 0 && axis1_mix_lds(c->K1, 1 << rsh) > 53 * 1024) --rsh;
+        while (rsh > 1 && axis1_mix_lds(c->K1, 1 << rsh) > 53 * 1024) --rsh;
         static bool attr = false;
         if (!attr) {
             (void)hipFuncSetAttribute((const void *)k_pme_axis1_mix, hipFuncAttributeMaxDynamicSharedMemorySize,

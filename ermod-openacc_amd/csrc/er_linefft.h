@@ -318,11 +318,13 @@ __global__ void __launch_bounds__(512) k_pme_spec2d_mix(int nslot, const SlotDes
 
 // Stage B for any K1 of small prime factors, 16 interleaved insertions: the
 // complex-to-real transform along axis 1 of RL = 2^rsh consecutive (x2, x3)
-// lines (T and phi are both contiguous over them).  Two insertions share one
-// complex transform of length K1: Z = X_a + i X_b over the whole Hermitian
-// spectrum gives phi_a and phi_b as its real and imaginary parts, for even
-// and odd K1 alike.  Each XCD sweeps one contiguous eighth of the blocks, so
-// that the two halves of a 128-byte line of T meet in one L2.
+// lines (T and phi are both contiguous over them), RL at least 2.  Two
+// neighbouring lines of one insertion share one complex transform of length
+// K1: Z = X_a + i X_b over the whole Hermitian spectrum gives phi_a and phi_b as
+// its real and imaginary parts, for even and odd K1 alike.  (Two insertions
+// in one transform would carry a non-finite one into the other.)
+// Each XCD sweeps one contiguous eighth of the blocks, so that the two halves
+// of a 128-byte line of T meet in one L2.
 __host__ __device__ constexpr size_t axis1_mix_lds(int K1, int RL)
 {
     return ((size_t)RL * 8 * (K1 | 1) + K1) * 8 + (((size_t)K1 * 2 + 7) / 8) * 8;
@@ -334,9 +336,9 @@ __global__ void __launch_bounds__(256) k_pme_axis1_mix(int nchunk, int K1, int n
                                                        const float2 *__restrict__ tws)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int H = K1 / 2 + 1, LS = K1 | 1, RL = 1 << rsh, NT = blockDim.x, tid = threadIdx.x;
-    const int NL = RL * 8;                              // complex lines of the block
-    float2 *Z = reinterpret_cast<float2 *>(smem);       // [RL][8 pairs][LS]
+    const int H = K1 / 2 + 1, LS = K1 | 1, RL = 1 << rsh, NP = RL >> 1, NT = blockDim.x, tid = threadIdx.x;
+    const int NL = NP * 16;                             // complex lines of the block
+    float2 *Z = reinterpret_cast<float2 *>(smem);       // [NP line pairs][16 insertions][LS]
     float2 *tw = Z + (size_t)NL * LS;                   // [K1]
     unsigned short *rv = reinterpret_cast<unsigned short *>(tw + K1);
     const int ngrp = (nline + RL - 1) >> rsh;
@@ -349,15 +351,15 @@ __global__ void __launch_bounds__(256) k_pme_axis1_mix(int nchunk, int K1, int n
         rv[k] = rev1[k];
     }
     __syncthreads();
-    // line r, pair p, m: X_a, X_b -> Z(m) and Z(K1 - m)
+    // line pair q, insertion p, m: X_a, X_b -> Z(m) and Z(K1 - m)
     for (int it = tid; it < H * NL; it += NT) {
-        const int r = it & (RL - 1), p = (it >> rsh) & 7, m = it >> (rsh + 3);
-        const int na = tile * 16 + 2 * p;
-        const bool in = l0 + r < nline;
-        const float2 *src = T + ((size_t)na * H + m) * nline + l0 + r;
-        float2 a = (in && na < nchunk) ? src[0] : make_float2(0.f, 0.f);
-        float2 b = (in && na + 1 < nchunk) ? src[(size_t)H * nline] : make_float2(0.f, 0.f);
-        float2 *z = Z + (r * 8 + p) * LS;
+        const int q = it & (NP - 1), p = (it >> (rsh - 1)) & 15, m = it >> (rsh + 3);
+        const int n = tile * 16 + p, la = l0 + 2 * q;
+        const bool live = n < nchunk && la < nline;
+        const float2 *src = T + ((size_t)n * H + m) * nline + la;
+        const float2 a = live ? src[0] : make_float2(0.f, 0.f);
+        const float2 b = live && la + 1 < nline ? src[1] : make_float2(0.f, 0.f);
+        float2 *z = Z + (q * 16 + p) * LS;
         if (m == 0 || 2 * m == K1) {  // their own mirror images: real
             z[rv[m]] = make_float2(a.x, b.x);
         } else {
@@ -367,12 +369,15 @@ __global__ void __launch_bounds__(256) k_pme_axis1_mix(int nchunk, int K1, int n
     }
     __syncthreads();
     line_dft(p1, Z, NL, mL, LS, 1, tw, tws);
-    // phi[line][x1][16]: eight pairs of one x1 are one 64-byte run
+    // phi[line][x1][16]: the 16 insertions of one x1 are one 64-byte run, two per thread
     float2 *dst = reinterpret_cast<float2 *>(phi + ((size_t)tile * nline + l0) * K1 * 16);
     const int nr = min(RL, nline - l0);
-    for (int r = 0; r < nr; ++r)
+    for (int q = 0; 2 * q < nr; ++q)
         for (int it = tid; it < K1 * 8; it += NT) {
             const int p = it & 7, x1 = it >> 3;
-            dst[(size_t)r * K1 * 8 + it] = Z[(r * 8 + p) * LS + x1];
+            const float2 *z = Z + (q * 16 + 2 * p) * LS + x1;
+            const float2 u = z[0], v = z[LS];
+            dst[(size_t)(2 * q) * K1 * 8 + it] = make_float2(u.x, v.x);
+            if (2 * q + 1 < nr) dst[(size_t)(2 * q + 1) * K1 * 8 + it] = make_float2(u.y, v.y);
         }
 }
