@@ -1925,22 +1925,22 @@ __global__ void __launch_bounds__(512) k_gather_brick(int K1, int K2, int K3, in
                     for (int c2 = 0; c2 < ORD; ++c2) {
                         const float4 p = pr[c3 % RB][c2];
                         const float w2 = t.w2[c2];
-                        zs.x += w2 * p.x;
-                        zs.y += w2 * p.y;
-                        zs.z += w2 * p.z;
-                        zs.w += w2 * p.w;
+                        zs.x = fmaf(w2, p.x, zs.x);
+                        zs.y = fmaf(w2, p.y, zs.y);
+                        zs.z = fmaf(w2, p.z, zs.z);
+                        zs.w = fmaf(w2, p.w, zs.w);
                     }
                     const float w3 = t.w3[c3];
-                    xs.x += w3 * zs.x;
-                    xs.y += w3 * zs.y;
-                    xs.z += w3 * zs.z;
-                    xs.w += w3 * zs.w;
+                    xs.x = fmaf(w3, zs.x, xs.x);
+                    xs.y = fmaf(w3, zs.y, xs.y);
+                    xs.z = fmaf(w3, zs.z, xs.z);
+                    xs.w = fmaf(w3, zs.w, xs.w);
                 }
                 const float w1 = t.w1[m];
-                ea.x += w1 * xs.x;
-                ea.y += w1 * xs.y;
-                ea.z += w1 * xs.z;
-                ea.w += w1 * xs.w;
+                ea.x = fmaf(w1, xs.x, ea.x);
+                ea.y = fmaf(w1, xs.y, ea.y);
+                ea.z = fmaf(w1, xs.z, ea.z);
+                ea.w = fmaf(w1, xs.w, ea.w);
             }
         }
         // every lane of the wave takes part in the exchanges (the XL x-lanes
@@ -2242,7 +2242,9 @@ __global__ void __launch_bounds__(ER_GS_NT) k_gather_stream(int K1, int K2, int 
 // behind the copies in flight into it, and here the planes read and the
 // planes written are always different ones.  Each wave waits for its own copies
 // before the barrier that ends the step.
-// Arithmetic as in k_gather_brick.  Two lanes per insertion quad share an atom
+// Arithmetic as in k_gather_brick, every fused product written out in both, so
+// that the chunk a run is cut into, which decides between them, changes no
+// bit.  Two lanes per insertion quad share an atom
 // (even and odd x offsets): four leave a quarter of their columns empty (1526 us
 // on the first shape below).  Bound by LDS reads (66 % of the cycles busy) where
 // atoms are dense, by the staging where they are sparse: 90 000 atoms x 700
@@ -2416,13 +2418,13 @@ __global__ void __launch_bounds__(ER_SW_NT) k_gather_sweep(int K1, int K2, int K
 #pragma unroll
                         for (int c2 = 0; c2 < ORD; ++c2) {
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) zs[e] += f[ORD + c2] * pr[c2][e];
+                            for (int e = 0; e < 4; ++e) zs[e] = fmaf(f[ORD + c2], pr[c2][e], zs[e]);
                         }
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) xs[e] += f[2 * ORD + c3] * zs[e];
+                        for (int e = 0; e < 4; ++e) xs[e] = fmaf(f[2 * ORD + c3], zs[e], xs[e]);
                     }
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) ea[e] += w1 * xs[e];
+                    for (int e = 0; e < 4; ++e) ea[e] = fmaf(w1, xs[e], ea[e]);
                 }
             }
             // the x-lanes of an atom, XL consecutive groups of LPP lanes; every
