@@ -2263,11 +2263,15 @@ template <int ORD> struct Sweep {
 };
 #define ER_SW_NT 1024
 // one row of planes or records into LDS: lane l's 16 bytes at base + off land at
-// LDS byte address lds + 16 l
+// LDS byte address lds + 16 l.  m0, which holds that address, is given back as
+// it was: the compiler may keep a value of its own there (and takes it for a
+// reserved register, which a clobber list cannot name).
 __device__ __forceinline__ void lds_copy16(const void *base, unsigned int off, unsigned int lds)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
+    unsigned int m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\t"
+                 "s_mov_b32 m0, %0"
+                 : "=&s"(m0)
                  : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(base)
                  : "memory");
 }
