@@ -3017,6 +3017,9 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
         if (lane == 0) take = atomicAdd(ctr, k);
         return __builtin_amdgcn_readfirstlane(take);
     };
+    // The lanes of a wave exchange values through LDS below: the wave runs its
+    // LDS accesses in order, the fence keeps the compiler to it.
+    auto exchanged = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
     for (int c = next(&nextL, 1); c < nlg; c = next(&nextL, 1)) {
         const int jm = __builtin_amdgcn_readfirstlane(cand[ER_PAIR_CAP - 1 - c]);
         const int b0 = molbeg[jm], b1 = molbeg[jm + 1];
@@ -3024,6 +3027,7 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
         for (int sb = 0; sb < pa.nslt; sb += ER_PAIR_SCAP) {  // 256 sites at a time (one block of them in LDS)
             const int se = min(pa.nslt, sb + ER_PAIR_SCAP);
             for (int st = lane; st < se - sb; st += 64) sums[wv][st] = 0.0f;
+            exchanged();
             for (int s0 = b0; s0 < b1; s0 += ER_SEG) {
                 const int at = min(s0 + w8, b1 - 1);
                 const bool atom = s0 + w8 < b1;
@@ -3064,7 +3068,9 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
                     if (w8 == 0 && s < se) sums[wv][s - sb] = es;
                 }
             }
+            exchanged();
             for (int st = lane; st < se - sb; st += 64) e += sums[wv][st];
+            exchanged();
         }
         for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
         if (lane == 0) U[urow + (size_t)jm * pa.NI] += e;
@@ -3104,6 +3110,7 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
                 nf += __popcll(mf);
                 nbk += __popcll(mb);
             }
+            exchanged();
             const int nfw = (nf + 63) & ~63, nlist = nfw + nbk;  // whole waves of either kind
             for (int l0 = 0; l0 < nlist; l0 += 64) {
                 const bool front = l0 < nfw;
@@ -3136,6 +3143,7 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
                     }
                 if (on) sums[wv][we * nsb + s] = e;
             }
+            exchanged();
             // the site sums of lane class g, added over g, g + GS, ...
             const int grp = lane / GS, gl = lane % GS;
             for (int w0 = 0; w0 < W; w0 += 64 / GS) {
@@ -3146,6 +3154,7 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
                 for (int off = GS / 2; off > 0; off >>= 1) e += __shfl_xor(e, off, 64);
                 if (gl == 0 && c0 + w0 + grp < ns) U[urow + (size_t)cand[c0 + w0 + grp] * pa.NI] += e;
             }
+            exchanged();
         }
     }
     // More candidates than the list holds: the search goes on where it stopped,
