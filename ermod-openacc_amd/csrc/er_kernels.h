@@ -2810,8 +2810,9 @@ __device__ __forceinline__ void pair_candidates(const PairArgs &pa, const FrameC
     const int span = min(2 * nreach + 1, pa.nc);  // distinct cells per axis
     const int lo = (span == pa.nc) ? 0 : -nreach;
     const int ncell = span * span * span;
-    for (; at.c < ncell; at.c += NT * pa.nsplit, at.p = 0) {
-        const int c = at.c;
+    bool on = true;  // nothing refused yet (an exit out of the loops would cost every launch)
+    int skip = at.p;
+    for (int c = at.c; c < ncell; c += NT * pa.nsplit, skip = 0) {
         const int dx = c % span, dy = (c / span) % span, dz = c / (span * span);
         // cx + lo + dx lies in [-nreach, nc + nreach) with nreach < nc (or lo = 0):
         // one conditional wrap
@@ -2819,7 +2820,7 @@ __device__ __forceinline__ void pair_candidates(const PairArgs &pa, const FrameC
         const unsigned int key = cell_key(qx, qy, qz, pa.nc);
         const unsigned int p0 = cstart[key], p1 = cstart[key + 1];
         // the cell's molecules four at a time: indices, then centres
-        for (unsigned int pb = p0 + at.p; pb < p1; pb += 4) {
+        for (unsigned int pb = p0 + skip; pb < p1; pb += 4) {
             int jk[4];
             float4 mk[4];
 #pragma unroll
@@ -2834,13 +2835,14 @@ __device__ __forceinline__ void pair_candidates(const PairArgs &pa, const FrameC
                 float ddx = m.x - ref.x, ddy = m.y - ref.y, ddz = m.z - ref.z;
                 min_image(fc, ddx, ddy, ddz);
                 const float lim = cut + m.w;
-                if (ddx * ddx + ddy * ddy + ddz * ddz <= lim * lim && !take(j)) {
-                    at.p = (int)(pb + k - p0);
-                    return;
+                if (ddx * ddx + ddy * ddy + ddz * ddz <= lim * lim && on && !take(j)) {
+                    on = false;
+                    at = {c, (int)(pb + k - p0)};
                 }
             }
         }
     }
+    if (on) at.c = 0x7fffffff;  // done: no cell left for a further call
 }
 
 // Pairs of the solutes of at most 8 sites, one (insertion, part) block per
@@ -3164,7 +3166,7 @@ k_pairs_many(PairArgs pa0, int blk0, int nslot, const SlotDesc *__restrict__ sd,
     // molecules come here and not their sums.  Rounds of the code above would
     // be the faster form, but around it the compiler keeps the loop's
     // constants in 26 more registers, a workgroup less per CU for every launch.
-    while (ncand > ER_PAIR_CAP) {  // uniform: no one adds to it between barriers
+    while (__builtin_expect(ncand > ER_PAIR_CAP, 0)) {  // uniform: no one adds to it between barriers
         __syncthreads();
         if (tid == 0) ncand = 0;
         __syncthreads();
