@@ -99,8 +99,7 @@ template <typename T> struct HBuf {
 }  // namespace
 
 // Scratch of er_run_noalloc: the split-K partial sums of edens/ecorr, in
-// device memory that the library never
-// allocates at run time.  Each GPU holds its own copy for the life of the
+// device memory that the library never allocates at run time.  Each GPU holds its own copy for the life of the
 // process.  In host code `scratch` names a host-side stand-in, not a device
 // address: kernels receive the per-device address that hipGetSymbolAddress
 // returns at er_create.  Every er_run_noalloc on one GPU shares the array,
@@ -635,7 +634,8 @@ extern "C" int er_create(const er_topology *topo, const er_params *prm, er_ctx *
     if (prm->splodr < 3 || prm->splodr > 10)
         return bad(fail(c, ER_E_UNSUPPORTED, "er_create: splodr must lie in 3..10"));
     // any grid: the compiled shapes run the four-step kernels, the others the
-    // direct-DFT ones, whose plane must fit a workgroup's LDS
+    // factored or (a prime factor above 7) the direct ones, whose plane must
+    // fit a workgroup's LDS (spec2d_gen_lds is the larger)
     for (int d = 0; d < 3; ++d)
         if (prm->ms[d] < std::max(16, 2 * prm->splodr) || prm->ms[d] > 512)
             return bad(fail(c, ER_E_UNSUPPORTED, "er_create: ms%dmax = %d outside %d..512", d + 1, prm->ms[d],
@@ -1489,7 +1489,7 @@ template <int NI> static hipError_t launch_axis1(er_ctx *c, int nch)
         // the factored kernel: the most lines per workgroup (64-byte runs of T
         // at eight) whose LDS still leaves three workgroups per CU, at least
         // the two that share a transform (71 KB at K1 = 512).  60 x 60 x
-        // 100, 300 insertions: 258 us (3.4 TB/s over T and phi) against 681 us direct.
+        // 100, 300 insertions: 240 us (3.7 TB/s over T and phi) against 681 us direct.
         int rsh = 3;
         while (rsh > 1 && axis1_mix_lds(c->K1, 1 << rsh) > 53 * 1024) --rsh;
         static bool attr = false;
@@ -1637,8 +1637,7 @@ template <int NI> static hipError_t launch_hist(er_ctx *c, int n_off, int nch)
 {
     // 512 threads per tile and slice for the batched path (more waves per CU
     // than 256 at the same slice count and global merge traffic); the plain
-    // path's single-insertion tiles keep 256 (its per-thread partials are
-    // reduced by one thread)
+    // path's single-insertion tiles keep 256
     const int NT = NI > 1 ? 512 : 256;
     const size_t nred = (size_t)NT / 64 * NI;  // per-wave partials
     const size_t lds = nred * sizeof(double) + (size_t)c->ermax * sizeof(float) +
@@ -1949,8 +1948,8 @@ static int upload_plan(er_ctx *c)
     return ER_OK;
 }
 
-// the split-K partials (ecorr, edens) of the run: the context's buffers, or in an er_run_noalloc call consecutive
-// ranges of the scratch array
+// the split-K partials (ecorr, edens) of the run: the context's buffers, or in
+// an er_run_noalloc call consecutive ranges of the scratch array
 struct AccPartials {
     double *part, *epart;
 };
@@ -2295,7 +2294,7 @@ static int run_slots(er_ctx *c, const std::vector<int> &todo, int mode)
         }
         for (const SlotDesc &d : P.desc) maxslt = std::max(maxslt, d.nslt);
         // four waves per insertion; few insertions of many sites take eight
-        // (a lone 150-site solute among 12 000 waters: 41 us in four, 30 us in eight)
+        // (a lone 150-site solute among 12 000 waters: 35 us in four, 31 us in eight)
         const int waves = maxslt > 32 && P.ntot <= 64 ? 8 : 4;
         const size_t nf = bare ? 0 : (size_t)P.nsite * (c->H + c->K2 + c->K3);
         const size_t nC = (size_t)P.ntot * c->ermax;

@@ -379,8 +379,8 @@ struct InsSource {
 // in the run).
 // Bound by the FP64 erf chain of the self energy: its pairs go round
 // ER_PI_PART partial sums, dealt to the threads and added in one order whatever
-// the wave count, so a lone 150-site solute can take eight waves (30 us;
-// 64 us for the sites and the self energy in four waves).
+// the wave count, so a lone 150-site solute can take eight waves (31 us, 35 in
+// four).
 #define ER_PI_ROWS 512   // sites held in LDS
 #define ER_PI_PART 1024  // partial sums of the self energy
 template <int ORD>
@@ -1618,7 +1618,9 @@ __global__ void __launch_bounds__(1024) k_sort_small(int nmol, const float4 *__r
     extern __shared__ __align__(16) unsigned int lcnt[];  // [ncell] cells, then [nbrick] bricks
     __shared__ unsigned int wsum[16];
     const int tid = threadIdx.x, nb = sg.nbrick;
-    unsigned int *bc = lcnt + ncell;  // ncell is a multiple of 64
+    // 16-byte aligned: ncell is a multiple of 64 wherever there are bricks (an
+    // open system has one cell and none)
+    unsigned int *bc = lcnt + ncell;
     for (int b = tid; b < ncell + nb; b += 1024) lcnt[b] = 0u;
     __syncthreads();
     float R = 0.0f;
@@ -2246,8 +2248,9 @@ __global__ void __launch_bounds__(ER_GS_NT) k_gather_stream(int K1, int K2, int 
 // that the chunk a run is cut into, which decides between them, changes no
 // bit.  Two lanes per insertion quad share an atom
 // (even and odd x offsets): four leave a quarter of their columns empty (1526 us
-// on the first shape below).  Bound by LDS reads (66 % of the cycles busy) where
-// atoms are dense, by the staging where they are sparse: 90 000 atoms x 700
+// on the first shape below).  No unit is full where atoms are dense (LDS 61 %,
+// VALU 41 %: a step holds fewer atoms than a pass has slots, and waves without
+// one wait at its barrier); the staging bounds it where they are sparse: 90 000 atoms x 700
 // insertions on 72^3 1410 -> 1386 us against a region per brick, 8 100 atoms x
 // 300 insertions in a slab of a 60 x 60 x 100 grid 677 -> 424 us; one plane
 // depth less per step (BZ = 2) 1527 and 509 us, 512 threads 1455 and 438 us.
@@ -2945,9 +2948,9 @@ __device__ __forceinline__ float row_shl(float v)
 //    reaches (one ballot over the clusters).
 // Skipped pairs lie beyond both cutoffs (triangle inequality on minimum
 // images, with a margin over FP32 rounding) and would add +0.
-// Bound by VALU and the LJ-table gathers of the pairs in reach.  A lane per
+// Bound by VALU issue (89 % of its slots).  A lane per
 // site looping over the atoms (the earlier form) left most lanes idle: 256
-// insertions of a 150-site solute among 200 000 atoms took 2112 us there, 1280 us
+// insertions of a 150-site solute among 200 000 atoms took 2112 us there, 1330 us
 // here; 250 insertions each of 9 to 45 sites among waters and 9-site molecules 800
 // and 545 us.
 __global__ void __launch_bounds__(256)

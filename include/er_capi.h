@@ -92,7 +92,7 @@ int er_create(const er_topology *topo, const er_params *prm, er_ctx **out);
 
 /* Replaces: enginit's mesh (engproc.F90:127-281).  uvmax/uvsoft: [numslv];
  * uvcrd: [sum(uvmax)] FP64 concatenated per species; escrd: [esmax] (only
- * read when selfcal = 1). */
+ * read when selfcal = 1).  A mesh that is refused changes nothing. */
 int er_set_mesh(er_ctx *c, const int32_t *uvmax, const int32_t *uvsoft,
                 const double *uvcrd, int32_t esmax, const double *escrd);
 
@@ -107,7 +107,7 @@ int er_set_solute(er_ctx *c, int32_t nsite, const int32_t *ljtype, const float *
  * processes every slot that has insertions, sharing the frame's
  * preparation.  nsite: [nsolute]; ljtype (1-based) and charge (x 18.22261721):
  * concatenated in solute order.  Resets every slot's accumulators; slot 1
- * is selected afterwards. */
+ * is selected afterwards.  Arguments that are refused change nothing. */
 int er_set_solutes(er_ctx *c, int32_t nsolute, const int32_t *nsite, const int32_t *ljtype,
                    const float *charge);
 
@@ -132,7 +132,9 @@ int er_set_frame_device(er_ctx *c, const float *sitepos_dev, const float *cell,
 /* Replaces: instslt('proc') x maxdst (engproc.F90:810-812) -- the caller
  * places the insertions.  sltpos: [3*nsite*nins] (insertion-major, i.e. the
  * sitepos extension slots of erdst/setconf.F90:607-611); stat_weight_solute:
- * [nins] or NULL for all 1. */
+ * [nins] or NULL for all 1.  sltpos_dev is a device pointer that stays valid
+ * until the next er_run() has completed; er_run fails where its allocation
+ * ends before the insertions do. */
 int er_set_insertions(er_ctx *c, int32_t nins, const float *sltpos,
                       const float *stat_weight_solute);
 int er_set_insertions_device(er_ctx *c, int32_t nins, const float *sltpos_dev,
@@ -218,7 +220,8 @@ int er_fetch(er_ctx *c, double *edens, double *ecorr, double *eself, double *sca
              float *minuv, float *maxuv, double *slnuv);
 
 /* Per-solute species sums of the last soln er_run (flceng, engproc.F90:918-932);
- * flceng: [numslv*nslt]. */
+ * flceng: [numslv*nslt], nslt that of the run (er_set_solute_molecules since
+ * then does not change it). */
 int er_get_flceng(er_ctx *c, double *flceng);
 
 /* Replaces: engclear (engproc.F90:321-340). */
