@@ -2218,15 +2218,14 @@ static hipError_t run_accumulate(er_ctx *c, AccRange ar)
     return hipGetLastError();
 }
 
-// Where a run's insertion coordinates lie: in the context's own buffer or in
-// memory of this device, which the kernels read in place; anywhere else (host
-// memory, another device's), which only a copy reads; or in an allocation that
-// ends before them.
-enum class InsAt { HERE, ELSEWHERE, SHORT };
-static InsAt insertions_at(const Slot &sl, size_t bytes)
+// Whether the kernels can read a run's insertion coordinates in place: in the
+// context's own buffer, or in an allocation of this device that holds all of
+// them.  Anything else is copied first: a copy reaches host memory and other
+// devices, and fails where an allocation is too short.
+static bool insertions_in_place(const Slot &sl, size_t bytes)
 {
     const float *p = sl.d_sltpos;
-    if (p == sl.d_sltpos_own.p && bytes <= sl.d_sltpos_own.n * sizeof(float)) return InsAt::HERE;
+    if (p == sl.d_sltpos_own.p && bytes <= sl.d_sltpos_own.n * sizeof(float)) return true;
     hipPointerAttribute_t at{};
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
@@ -2235,11 +2234,10 @@ static InsAt insertions_at(const Slot &sl, size_t bytes)
         at.type != hipMemoryTypeDevice || at.device != dev ||
         hipMemGetAddressRange(&base, &size, const_cast<float *>(p)) != hipSuccess) {
         (void)hipGetLastError();
-        return InsAt::ELSEWHERE;
+        return false;
     }
     const size_t off = (size_t)(reinterpret_cast<const char *>(p) - static_cast<const char *>(base));
-    if (off + bytes > size) return InsAt::SHORT;
-    return reinterpret_cast<uintptr_t>(p) % alignof(float) ? InsAt::ELSEWHERE : InsAt::HERE;
+    return off + bytes <= size && reinterpret_cast<uintptr_t>(p) % alignof(float) == 0;
 }
 
 // one run over the solutes `todo` of the frame: per-insertion preparation,
@@ -2266,13 +2264,9 @@ static int run_slots(er_ctx *c, const std::vector<int> &todo, int mode)
     // the insertions' coordinates: in place, or copied end to end
     bool copied = nslot > ER_INS_PTRS;
     if (!soln)
-        for (int i = 0; i < nslot; ++i) {
+        for (int i = 0; i < nslot && !copied; ++i) {
             const Slot &sl = c->slots[P.order[i]];
-            const InsAt at = insertions_at(sl, (size_t)P.desc[i].nins * sl.nslt * 3 * sizeof(float));
-            if (at == InsAt::SHORT)
-                return fail(c, ER_E_HIP, "er_run: the device memory of solute %d's insertions ends before them",
-                            P.order[i] + 1);
-            copied = copied || at == InsAt::ELSEWHERE;
+            copied = !insertions_in_place(sl, (size_t)P.desc[i].nins * sl.nslt * 3 * sizeof(float));
         }
     {
         ProfScope ps(c, ER_K_PREP);
